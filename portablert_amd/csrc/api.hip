@@ -333,7 +333,7 @@ static int chunked_pass(prt_ctx *c, const float *rays, uint64_t n, uint32_t mask
 			if (e == hipSuccess) e = hipStreamWaitEvent(c->stream, c->ev_in[b], 0);
 			if (e != hipSuccess) return hip_fail(c, e, "nearest_hits: ray upload");
 			if (int r = trace_common(c, d_rays + 6 * first, cnt, mask, d_out + first * stride, c->stream)) return r;
-			e = hipMemcpyAsync(c->chunk_err.as<uint32_t>() + i, c->ts.counter.as<uint32_t>() + 8, sizeof(uint32_t),
+			e = hipMemcpyAsync(c->chunk_err.as<uint32_t>() + i, prt::trace_error_word(c->ts), sizeof(uint32_t),
 			                   hipMemcpyDeviceToDevice, c->stream);
 			if (e == hipSuccess) e = hipEventRecord(c->ev_tr[b], c->stream);
 			if (e == hipSuccess) e = hipStreamWaitEvent(c->s_out, c->ev_tr[b], 0);
@@ -460,7 +460,7 @@ int prt_mi355x_synchronize(prt_ctx *c) {
 	uint32_t flags = 0, flags_na = 0;
 	if (e == hipSuccess) e = prt::trace_errors(c->ts, c->stream, &flags);
 	if (e == hipSuccess && c->used_noalloc)
-		e = prt::trace_errors_at(c->ts, static_cast<const uint32_t *>(prt::noalloc_scratch(c->device)), c->stream,
+		e = prt::trace_errors_at(c->ts, prt::noalloc_scratch(c->device), c->stream,
 		                         &flags_na);
 	flags |= flags_na;
 	if (e != hipSuccess) return hip_fail(c, e, "synchronize");

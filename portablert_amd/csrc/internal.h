@@ -144,13 +144,19 @@ struct TraceStats {
 };
 
 struct TraceScratch {
-	DevBuf counter;  // work counter + stats
+	static constexpr int kSets = 3, kSetWords = 16;  // 0 and 1 alternate, 2 serves captured launches
+	DevBuf counter;  // kSets sets of work counter, statistics and error flags
 	DevBuf spill;    // per-thread stack spill
 	int n_cus = 0;
-	uint32_t *host_err = nullptr;  // pinned copy of the last launch's error flags
+	int next_set = 0, last_set = 0;
+	bool clean = false;  // set next_set is all 0 once the work enqueued so far has run
+	unsigned long long *host_err = nullptr;  // pinned copy of the sets
+	unsigned long long *set(int k) const { return counter.as<unsigned long long>() + k * kSetWords; }
 };
 
-// Reads the error flags of the last traversal launched with `s` (synchronises `st`).
+// Error flags of the last launch with `s`, as a device address valid until the launch after it.
+const uint32_t *trace_error_word(const TraceScratch &s);
+// Reads the error flags of the last traversals launched with `s` (synchronises `st`).
 hipError_t trace_errors(TraceScratch &s, hipStream_t st, uint32_t *flags);
 
 // Traces n device rays against `b`, writing HitReg records at `out` (device) with the layout
@@ -193,6 +199,6 @@ void *noalloc_scratch(int device);
 hipError_t trace_bvh8_noalloc(const Bvh8 &b, TraceScratch &s, const TraceParams &p, const float *rays, uint64_t n,
                               uint32_t mask, void *out, hipStream_t st, void *scratch_ptr, uint64_t *need_bytes);
 // Error flags of the last launch that used `counter` (synchronises st).
-hipError_t trace_errors_at(TraceScratch &s, const uint32_t *counter, hipStream_t st, uint32_t *flags);
+hipError_t trace_errors_at(TraceScratch &s, const void *counter, hipStream_t st, uint32_t *flags);
 
 }  // namespace prt

@@ -34,7 +34,8 @@ struct KArgs {
 	const TriRec *tris;
 	const float *rays;
 	uint8_t *out;
-	uint32_t *counter;      // [0] work counter, [1..3] stats
+	unsigned long long *counter;  // kCounters words (C_*), all 0 at the start of the launch
+	unsigned long long *next;     // another set, cleared here for the launch that follows, or null
 	uint2 *spill;           // spill_depth entries per launched thread
 	uint64_t n_rays;
 	uint32_t n_nodes;
@@ -63,6 +64,27 @@ struct KArgs {
 	const float2 *scene_info;
 };
 
+// Words of a launch's counters.
+enum : int {
+	C_WORK = 0,       // next ray (or tile) of the main pass
+	C_NODES = 1,      // statistics
+	C_TRIS = 2,
+	C_LEAVES = 3,
+	C_ERR = 4,        // low 32 bits: error flags, high 32 bits: 1 once a ray was left to the second pass
+	C_NPHASE = 5,
+	C_TPHASE = 6,
+	C_CULLED = 7,
+	C_WORK_REST = 8,  // next ray (or tile) of the second pass
+	kCounters = 9
+};
+
+// Quantized nodes are traversed in two launches: kFast takes the rays of the one-fma node test
+// and leaves the others (d_x = 0, magnitudes out of its range) to kRest, whose waves end at once
+// where there are none, else go through all rays again and take those. One kernel for both held
+// the reference formula's registers against every ray: at the plain mode's 64 it spilled 10, and
+// with the treatment of d_x = 0 (child_slab) 58. kAll: fp32 nodes, one node test for every ray.
+enum Pass : int { kAll = 0, kFast = 1, kRest = 2 };
+
 // kWatertight: the plain traversal with the watertight leaf test (wt_candidate), no culling.
 // kSeeded searches the best predicted cluster first, kSeededMulti the best 2..4.
 enum : int { kPlain = 0, kSeeded = 1, kBatch = 2, kWatertight = 3, kSeededMulti = 4 };
@@ -71,18 +93,25 @@ constexpr uint32_t kInvalid = 0xFFFFFFFFu;
 
 // Per-lane ray state.
 struct Ray {
-	float o[3], d[3], inv[3];
+	float o[3], d[3];
+	float inv[3];      // 1/d, with +-kFlat in the place of +-inf where the one-fma node test is used
 	float tb, ub, vb;
 	uint32_t idb;
-	float abs_margin;  // margin_abs / |d|
-	bool degen;        // some 1/d is infinite: axis-parallel handling in node tests
-	bool patho;        // non-finite origin or NaN direction: every node passes
-	bool fast;         // |1/d| and |o| below 2^60 in a scene within 2^60: one-fma node bounds
+	float abs_margin;  // margin_abs / |d|; infinite: this ray is not culled by distance
+	bool mine;         // this launch traces the ray (Pass)
+	bool odd;          // some 1/d or o is not finite (child_slab)
+	bool never;        // no triangle can be hit: NaN in origin or direction, or no direction
 };
 
-__device__ __forceinline__ void load_ray(const float *rays, uint64_t idx, float margin_abs, bool fast_scene,
-                                         Ray &r) {
-	const float *p = rays + 6 * idx;  // 4-byte aligned AoS records of 24 bytes
+// Stands for 1/0 in the one-fma node test. A box around o_k on a zero axis then spans at least
+// +-2^42 (|p| + |o| + extent) there (the test's own margin, 2^-18 |1/d|), which holds every t of
+// the other axes (|t| <= 2^30 times the same lengths); a box that o_k lies outside of by more than
+// 2^-18 of its coordinates is left before any of them. All products stay below 2^127.
+constexpr float kFlat = 0x1p60f;
+
+template <int PASS, bool WT>
+__device__ __forceinline__ void load_ray(const KArgs &a, uint64_t idx, float margin_abs, bool fast_scene, Ray &r) {
+	const float *p = a.rays + 6 * idx;  // 4-byte aligned AoS records of 24 bytes
 #pragma unroll
 	for (int k = 0; k < 3; ++k) {
 		r.o[k] = p[k];
@@ -90,21 +119,35 @@ __device__ __forceinline__ void load_ray(const float *rays, uint64_t idx, float 
 	}
 #pragma unroll
 	for (int k = 0; k < 3; ++k) r.inv[k] = 1.0f / r.d[k];  // IEEE division, as the reference
-	r.degen = !(__builtin_isfinite(r.inv[0]) && __builtin_isfinite(r.inv[1]) && __builtin_isfinite(r.inv[2]));
-	r.patho = !(__builtin_isfinite(r.o[0]) && __builtin_isfinite(r.o[1]) && __builtin_isfinite(r.o[2])) ||
-	          __builtin_isnan(r.d[0]) || __builtin_isnan(r.d[1]) || __builtin_isnan(r.d[2]);
-	// |1/d| below 2^30 (every |d_k| above 2^-30), |o| below 2^60 in a scene within 2^60
+	// every |d_k| 0 or above 2^-30 (|1/d| below 2^30), |o| below 2^60 in a scene within 2^60
 	const float big = 0x1p60f, inv_big = 0x1p30f;
-	r.fast = fast_scene && !r.degen && !r.patho && fabsf(r.inv[0]) < inv_big && fabsf(r.inv[1]) < inv_big &&
-	         fabsf(r.inv[2]) < inv_big && fabsf(r.o[0]) < big && fabsf(r.o[1]) < big && fabsf(r.o[2]) < big;
+	const bool zero[3] = {r.d[0] == 0.0f, r.d[1] == 0.0f, r.d[2] == 0.0f};
+	bool nan = false, in_range = fast_scene;
+#pragma unroll
+	for (int k = 0; k < 3; ++k) {
+		nan |= __builtin_isnan(r.o[k]) || __builtin_isnan(r.d[k]);
+		in_range &= (zero[k] || fabsf(r.inv[k]) < inv_big) && fabsf(r.o[k]) < big;
+	}
+	// With NaN in the origin or the direction every t is NaN, which never wins; without a
+	// direction every determinant is 0 (Moller-Trumbore) or NaN (the watertight test).
+	r.never = nan || (zero[0] && zero[1] && zero[2]);
+	const bool fast = in_range && !zero[0];  // d_x = 0: the reference formula (child_slab)
+	r.mine = PASS == kFast ? fast || r.never : !(fast || r.never);
 	// margin_abs / |d|, rounded up (1 + 2^-20 covers the reciprocal square root's error). An
 	// infinite margin turns distance culling off for this ray: culling is exact only for rays
-	// with every direction component within [2^-30, 2^30] (|d|^2 <= 2^60 bounds them above) and
-	// |o| < 2^60 (cull_unsafe in common.h), i.e. fast rays; other rays (zero direction
-	// components, huge or tiny values) traverse without it.
+	// with every direction component 0 or within [2^-30, 2^30] (|d|^2 <= 2^60 bounds them above)
+	// and |o| < 2^60 (cull_unsafe in common.h; a zero component makes its products exactly 0, so
+	// the bound there holds); other rays (huge or tiny values) traverse without it.
 	const float len2 = r.d[0] * r.d[0] + r.d[1] * r.d[1] + r.d[2] * r.d[2];
-	r.abs_margin = (r.fast && len2 <= 0x1p60f) ? margin_abs * (__builtin_amdgcn_rsqf(len2) * (1.0f + 0x1p-20f))
-	                                           : __builtin_inff();
+	r.abs_margin = ((a.cull || WT) && in_range && len2 <= 0x1p60f)
+	                   ? margin_abs * (__builtin_amdgcn_rsqf(len2) * (1.0f + 0x1p-20f))
+	                   : __builtin_inff();
+	r.odd = !(__builtin_isfinite(r.inv[0]) && __builtin_isfinite(r.inv[1]) && __builtin_isfinite(r.inv[2]) &&
+	          __builtin_isfinite(r.o[0]) && __builtin_isfinite(r.o[1]) && __builtin_isfinite(r.o[2]));
+	if (PASS == kFast) {
+#pragma unroll
+		for (int k = 1; k < 3; ++k) r.inv[k] = zero[k] ? copysignf(kFlat, r.d[k]) : r.inv[k];
+	}
 	r.tb = __builtin_inff();
 	r.ub = r.vb = 0.0f;
 	r.idb = kInvalid;
@@ -119,12 +162,35 @@ __device__ __forceinline__ float cull_limit(const Ray &r, const KArgs &a) {
 // Conservative slab test of one child box [lo, hi]. Returns the entry distance (tmin), or NaN
 // when the box is rejected. WIDE (the watertight mode): the interval is widened by 2^-20 of its
 // end points, so that a ray through a box corner (a vertex shared by several triangles) is not
-// rejected by the rounding of tmin and tmax.
+// rejected by the rounding of tmin and tmax. `flagged`: the subtree holds an ill-conditioned
+// triangle (cull_unsafe).
+//
+// A ray with d_x = 0 whose origin lies exactly on the low x side of a triangle's own box meets
+// 0 * inf on the x axis, and the exact slab test of that triangle then passes outright, wherever
+// the box lies on the other axes and also behind the origin (bvh.hpp:210-217 with
+// std::max/std::min argument order). Only the leaf test can reject it, so every box that holds
+// o_x has to pass as far as the leaf test's error reaches: everywhere where that error is not
+// bounded (rays that are not culled by distance, flagged subtrees), else where the ray's line,
+// not only the part ahead, comes within 2^-10 of the coordinates' magnitude. The leaf test's
+// (u, v) place a hit of an unflagged triangle within 5 rho 2^-24 of these lengths, rho as in
+// cull_unsafe, so the pairs covered are those the culling margin covers (rho <= 2^13 / 5); the
+// watertight test's sheared vertices are within 2^-21 of them for every triangle.
+struct SlabRay {
+	float o[3], inv[3];
+	bool odd;   // some 1/d or o is not finite
+	bool line;  // d_x = 0, and the leaf test's error is bounded as above
+};
+
+__device__ __forceinline__ SlabRay slab_ray(const Ray &r) {
+	return {{r.o[0], r.o[1], r.o[2]}, {r.inv[0], r.inv[1], r.inv[2]}, r.odd, r.d[0] == 0.0f && r.abs_margin < __builtin_inff()};
+}
+
 template <bool WIDE = false>
-__device__ __forceinline__ float child_slab(const Ray &r, const float lo[3], const float hi[3], float limit) {
+__device__ __forceinline__ float child_slab(const SlabRay &r, const float lo[3], const float hi[3], float limit,
+                                            bool flagged = false) {
 #pragma clang fp contract(off)
 	float amin[3], amax[3];
-	bool poison = false;
+	bool pass = false, line = false;
 #pragma unroll
 	for (int k = 0; k < 3; ++k) {
 		const float t1 = (lo[k] - r.o[k]) * r.inv[k];
@@ -132,25 +198,35 @@ __device__ __forceinline__ float child_slab(const Ray &r, const float lo[3], con
 		amin[k] = fminf(t1, t2);
 		amax[k] = fmaxf(t1, t2);
 	}
-	if (r.degen) {
-		// 1/d infinite on an axis: a box side through the origin gives NaN in the exact test.
-		// Treat any box containing the origin's coordinate on that axis as unbounded there;
-		// on the x axis such a NaN makes the exact test pass outright (bvh.hpp:210-217 with
-		// std::max/std::min argument order), so the box must pass.
+	if (r.odd) {
+		// 1/d infinite on an axis: a box side through the origin gives NaN in the exact test, and a
+		// box containing the origin's coordinate on that axis is unbounded there.
+		const bool x_in = !__builtin_isfinite(r.inv[0]) && lo[0] <= r.o[0] && r.o[0] <= hi[0];
+		line = x_in && r.line;
+		pass = (x_in && (!line || flagged)) ||  // an infinite origin: every node passes
+		       !(__builtin_isfinite(r.o[0]) && __builtin_isfinite(r.o[1]) && __builtin_isfinite(r.o[2]));
+		if (x_in) {
+			amin[0] = -__builtin_inff();
+			amax[0] = __builtin_inff();
+		}
 #pragma unroll
-		for (int k = 0; k < 3; ++k) {
-			if (!__builtin_isfinite(r.inv[k]) && lo[k] <= r.o[k] && r.o[k] <= hi[k]) {
+		for (int k = 1; k < 3; ++k) {
+			const float tol = line ? 0x1p-10f * (fabsf(lo[k]) + fabsf(hi[k]) + fabsf(r.o[k])) : 0.0f;
+			if (__builtin_isfinite(r.inv[k])) {
+				amin[k] -= tol * fabsf(r.inv[k]);
+				amax[k] += tol * fabsf(r.inv[k]);
+			} else if (lo[k] - tol <= r.o[k] && r.o[k] <= hi[k] + tol) {
 				amin[k] = -__builtin_inff();
 				amax[k] = __builtin_inff();
-				if (k == 0) poison = true;
 			}
 		}
 	}
 	const float tmin = fmaxf(fmaxf(amin[0], amin[1]), amin[2]);
 	const float tmax = fminf(fminf(amax[0], amax[1]), amax[2]);
-	if (poison || r.patho) return -__builtin_inff();
-	const float slack = WIDE ? 0x1p-20f * (fabsf(tmin) + fabsf(tmax)) : 0.0f;
-	const bool hit = (tmax >= -slack) && (tmin <= tmax + slack) && (tmin <= limit);
+	if (pass) return -__builtin_inff();
+	float slack = WIDE ? 0x1p-20f * (fabsf(tmin) + fabsf(tmax)) : 0.0f;
+	if (WIDE && !__builtin_isfinite(slack)) slack = 0.0f;  // a zero axis: inside or outside, exactly
+	const bool hit = (line || tmax >= -slack) && (tmin <= tmax + slack) && (tmin <= limit);
 	return hit ? tmin : __builtin_nanf("");
 }
 
@@ -239,15 +315,11 @@ struct NodeHits {
 // rejects, so such a box is never culled (and is visited before its siblings).
 constexpr uint32_t kKeyNoCull = 0x00800000u;
 
-// Tests the children of one node (fast_ok selects the one-fma bound evaluation). Slots whose bit
+// Tests the children of one node (PASS kFast: by the one-fma bound evaluation). Slots whose bit
 // is set in the node's never-cull mask pass whenever the box is hit, at any distance, and take
 // the key kKeyNoCull | slot; the other slots of such a node are tested without the limit and
 // culled only when popped. `ncull_q` is the quantized node array, which holds the mask of
 // both formats (byte 15 of node idx).
-template <class Node, bool NC, bool WIDE>
-__device__ __forceinline__ void test_children(const Node *nodes, const NodeQ *ncull_q, uint32_t idx, const Ray &r,
-                                              float limit, bool fast_ok, NodeHits &h);
-
 // Byte k of a little-endian dword pair, as a float (one v_cvt_f32_ubyteN when k is constant).
 __device__ __forceinline__ float byte_f(const uint32_t w[2], int k) {
 	return static_cast<float>((w[k >> 2] >> (8 * (k & 3))) & 0xFFu);
@@ -263,13 +335,13 @@ __device__ __forceinline__ void no_cull_keys(uint32_t key[8], uint32_t ncull) {
 
 // NC = false: the scene has no flagged triangle (every mask is 0) and the masks are not read.
 // WIDE: widened reference-formula intervals (child_slab).
-template <class Node, bool NC, bool WIDE>
+template <class Node, bool NC, bool WIDE, int PASS>
 struct ChildTest;
 
-template <bool NC, bool WIDE>
-struct ChildTest<NodeQ, NC, WIDE> {
+template <bool NC, bool WIDE, int PASS>
+struct ChildTest<NodeQ, NC, WIDE, PASS> {
 static __device__ __forceinline__ void run(const NodeQ *nodes, const NodeQ * /*ncull_q*/, uint32_t idx, const Ray &r,
-                                           float limit, bool fast_ok, NodeHits &h) {
+                                           float limit, NodeHits &h) {
 	const uint4 *src = reinterpret_cast<const uint4 *>(nodes + idx);
 	const uint4 w0 = src[0], w1 = src[1], w2 = src[2], w3 = src[3], w4 = src[4];
 	const float p[3] = {__uint_as_float(w0.x), __uint_as_float(w0.y), __uint_as_float(w0.z)};
@@ -290,9 +362,9 @@ static __device__ __forceinline__ void run(const NodeQ *nodes, const NodeQ * /*n
 	// within 8 * 2^-24 * |1/d_a| * (255 * 2^e_a + |p_a| + |o_a|) of the real value, so moving the
 	// near plane in and the far plane out by 2^-18 times that amount keeps every fast interval
 	// around the interval the reference formula gives for the same dequantized box (which the
-	// builder already rounded outward). fast_ok guarantees |1/d|, |o| and the scene coordinates
+	// builder already rounded outward). A fast ray guarantees |1/d|, |o| and the scene coordinates
 	// are below 2^60, so none of these values overflows; other rays take the reference formula.
-	if (fast_ok) {
+	if constexpr (PASS == kFast) {
 		// a slot is used iff its meta byte is not 0xFF, i.e. its byte of the complement is not 0
 		const uint32_t unused_lo = ~meta_lo, unused_hi = ~meta_hi;
 		float step[3], bnear[3], bfar[3];
@@ -333,7 +405,8 @@ static __device__ __forceinline__ void run(const NodeQ *nodes, const NodeQ * /*n
 		sort8(h.key);
 		return;
 	}
-	// Reference formula on the dequantized box (also the path of the exact mode).
+	// Reference formula on the dequantized box.
+	const SlabRay sr = slab_ray(r);
 #pragma unroll
 	for (int k = 0; k < 8; ++k) {
 		const uint32_t meta = ((k < 4 ? meta_lo : meta_hi) >> (8 * (k & 3))) & 0xFFu;
@@ -345,7 +418,7 @@ static __device__ __forceinline__ void run(const NodeQ *nodes, const NodeQ * /*n
 			lo[ax] = fmaf(static_cast<float>(bl), s[ax], p[ax]);
 			hi[ax] = fmaf(static_cast<float>(bh), s[ax], p[ax]);
 		}
-		const float tmin = child_slab<WIDE>(r, lo, hi, ncull != 0u ? __builtin_inff() : limit);
+		const float tmin = child_slab<WIDE>(sr, lo, hi, ncull != 0u ? __builtin_inff() : limit, (ncull >> k) & 1u);
 		const bool hit = meta != kMetaEmpty && !__builtin_isnan(tmin);
 		h.key[k] = hit ? sort_key(tmin, k) : kMiss;
 	}
@@ -354,10 +427,10 @@ static __device__ __forceinline__ void run(const NodeQ *nodes, const NodeQ * /*n
 }
 };
 
-template <bool NC, bool WIDE>
-struct ChildTest<NodeF, NC, WIDE> {
+template <bool NC, bool WIDE, int PASS>
+struct ChildTest<NodeF, NC, WIDE, PASS> {
 static __device__ __forceinline__ void run(const NodeF *nodes, const NodeQ *ncull_q, uint32_t idx, const Ray &r,
-                                           float limit, bool /*fast_ok*/, NodeHits &hh) {
+                                           float limit, NodeHits &hh) {
 	const NodeF *n = nodes + idx;
 	const uint4 h = *reinterpret_cast<const uint4 *>(n);
 	const uint32_t ncull = NC ? reinterpret_cast<const uint32_t *>(ncull_q + idx)[3] >> 24 : 0u;
@@ -380,7 +453,7 @@ static __device__ __forceinline__ void run(const NodeF *nodes, const NodeQ *ncul
 		const uint32_t meta = ((k < 4 ? h.z : h.w) >> (8 * (k & 3))) & 0xFFu;
 		const float l[3] = {lo[0][k], lo[1][k], lo[2][k]};
 		const float u[3] = {hi[0][k], hi[1][k], hi[2][k]};
-		const float tmin = child_slab<WIDE>(r, l, u, ncull != 0u ? __builtin_inff() : limit);
+		const float tmin = child_slab<WIDE>(slab_ray(r), l, u, ncull != 0u ? __builtin_inff() : limit, (ncull >> k) & 1u);
 		const bool hit = meta != kMetaEmpty && !__builtin_isnan(tmin);
 		hh.key[k] = hit ? sort_key(tmin, k) : kMiss;
 	}
@@ -388,12 +461,6 @@ static __device__ __forceinline__ void run(const NodeF *nodes, const NodeQ *ncul
 	sort8(hh.key);
 }
 };
-
-template <class Node, bool NC, bool WIDE>
-__device__ __forceinline__ void test_children(const Node *nodes, const NodeQ *ncull_q, uint32_t idx, const Ray &r,
-                                              float limit, bool fast_ok, NodeHits &h) {
-	ChildTest<Node, NC, WIDE>::run(nodes, ncull_q, idx, r, limit, fast_ok, h);
-}
 
 // Lane 0's value in every lane, as a wave-uniform (scalar) value; every lane of the wave must be
 // active.
@@ -413,10 +480,14 @@ __device__ __forceinline__ void write_record(const KArgs &a, uint64_t ray_idx, c
 	write_any(a.mask, a.out + ray_idx * a.stride, h, r.o, r.d);
 }
 
-template <bool WT>
+template <bool WT, int PASS>
 __device__ __forceinline__ void test_leaf(const TriRec *tris, uint32_t entry, Ray &r) {
 	const uint32_t first = leaf_first(entry);
 	const uint32_t count = leaf_count(entry);
+	float inv[3];  // 1/d as the reference has it (kFast: y and z may hold kFlat)
+#pragma unroll
+	for (int k = 0; k < 3; ++k)
+		inv[k] = PASS == kFast && k > 0 && r.d[k] == 0.0f ? copysignf(__builtin_inff(), r.d[k]) : r.inv[k];
 	for (uint32_t m = 0; m < count; ++m) {
 		const uint4 *src = reinterpret_cast<const uint4 *>(tris + first + m);
 		const uint4 a = src[0], b = src[1], c = src[2];
@@ -425,7 +496,7 @@ __device__ __forceinline__ void test_leaf(const TriRec *tris, uint32_t entry, Ra
 		                    __uint_as_float(b.z), __uint_as_float(b.w), __uint_as_float(c.x)};
 		const uint32_t id = c.y;
 		float t, u, vv;
-		const bool cand = WT ? wt_candidate(v, r.o, r.d, r.inv, t, u, vv) : exact_candidate(v, r.o, r.d, r.inv, t, u, vv);
+		const bool cand = WT ? wt_candidate(v, r.o, r.d, inv, t, u, vv) : exact_candidate(v, r.o, r.d, inv, t, u, vv);
 		if (cand && better(t, id, r.tb, r.idb)) {
 			r.tb = t;
 			r.ub = u;
@@ -436,19 +507,24 @@ __device__ __forceinline__ void test_leaf(const TriRec *tris, uint32_t entry, Ra
 }
 
 // Waves per SIMD the register allocation must allow. Quantized nodes with an 8-entry LDS stack
-// (4 KB per wave): 8 for the plain mode, i.e. at most 64 VGPRs; the traversal is partly
-// latency-bound (dependent node fetches) and the extra waves hide more of it than the few
-// spilled registers cost. The seeded and batch modes carry more state per lane (seed clusters,
-// scene tiles) and spill more at 64 VGPRs: they run at 7 waves (72 VGPRs). Spills inside the
-// loop are costly here: the multi-seed state (three more entries, their flags) spills 14
-// registers at 72 VGPRs, and the one-seed mode, which carries one entry, runs 10% faster with
-// 2. A 16-entry stack allows 5 waves by LDS alone. The fp32 node test needs about 100 VGPRs
+// (4 KB per wave): 8 for the plain mode, i.e. at most 64 VGPRs, which it keeps to without a spill;
+// the traversal is partly latency-bound (dependent node fetches) and the extra waves hide more of
+// it. The other modes carry more state per lane (seed clusters, scene tiles) and would spill
+// 2 to 5 registers at 64: they run at 7 waves (72 VGPRs, no spill). Spills inside the loop cost far
+// more than a wave of occupancy: the batch step took 8.92 ms at 64 VGPRs with 5 of them, 8.22 ms
+// at 72. A 16-entry stack allows 5 waves by LDS alone. The fp32 node test needs about 100 VGPRs
 // and is left to the compiler (1 = no constraint).
-template <class Node, int S, int MODE>
-constexpr int kWavesPerEu = std::is_same<Node, NodeQ>::value ? (S == 8 ? (MODE == kPlain ? 8 : 7) : 5) : 1;
+template <int S, int MODE, int PASS>
+constexpr int kWavesPerEu = PASS == kFast ? (S == 8 ? (MODE == kPlain ? 8 : 7) : 5) : 1;
 
-template <class Node, int S, int B, bool COUNT, int MODE, bool NC>
-__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<Node, S, MODE>))) void k_trace(KArgs a) {
+template <class Node, int S, int B, bool COUNT, int MODE, bool NC, int PASS>
+__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<S, MODE, PASS>))) void k_trace(KArgs a) {
+	static_assert(std::is_same<Node, NodeF>::value == (PASS == kAll), "fp32 nodes take one pass");
+	unsigned long long *work = a.counter + (PASS == kRest ? C_WORK_REST : C_WORK);
+	uint32_t *flags = reinterpret_cast<uint32_t *>(a.counter + C_ERR);  // [0] errors, [1] rays left to kRest
+	if (PASS == kRest && flags[1] == 0u) return;
+	if (PASS != kRest && blockIdx.x == 0 && threadIdx.x < kCounters && a.next) a.next[threadIdx.x] = 0ull;
+	bool told = false;  // this wave has reported a ray left to kRest
 	constexpr bool MULTI = MODE == kSeededMulti, SEEDED = MODE == kSeeded || MULTI, BATCH = MODE == kBatch;
 	__shared__ uint2 lds[S * B];
 	const Node *nodes = static_cast<const Node *>(a.nodes);
@@ -488,7 +564,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<N
 		if (n_need != 0u && !exhausted && (n_need >= a.refill || n_need == __popcll(__ballot(true)))) {
 			if (chunk_next >= chunk_end && BATCH) {
 				uint64_t tix = 0;
-				if (lane == 0) tix = atomicAdd(reinterpret_cast<unsigned long long *>(a.counter), 1ull);
+				if (lane == 0) tix = atomicAdd(work, 1ull);
 				tix = uniform64(tix);
 				if (tix < a.n_tiles) {
 					const uint4 tl = a.tiles[tix];
@@ -502,8 +578,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<N
 				}
 			} else if (chunk_next >= chunk_end) {
 				uint64_t base = 0;
-				if (lane == 0) base = atomicAdd(reinterpret_cast<unsigned long long *>(a.counter),
-				                                static_cast<unsigned long long>(a.chunk));
+				if (lane == 0) base = atomicAdd(work, static_cast<unsigned long long>(a.chunk));
 				base = uniform64(base);
 				chunk_next = base;
 				chunk_end = base + a.chunk < a.n_rays ? base + a.chunk : a.n_rays;
@@ -518,18 +593,19 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<N
 			                                                __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(need), 0u));
 			if (!active && rank < avail) {
 				ray_idx = chunk_next + rank;
-				active = true;
 				if (BATCH) {
 					const float2 si = a.scene_info[chunk_scene];
-					load_ray(a.rays, ray_idx, si.x, si.y != 0.0f, r);
+					load_ray<PASS, MODE == kWatertight>(a, ray_idx, si.x, si.y != 0.0f, r);
 					cur = chunk_scene;
 				} else {
-					load_ray(a.rays, ray_idx, a.margin_abs, a.fast_scene != 0, r);
-					cur = a.n_nodes > 0 ? 0u : kInvalid;
+					load_ray<PASS, MODE == kWatertight>(a, ray_idx, a.margin_abs, a.fast_scene != 0, r);
+					cur = 0u;
 				}
+				if (r.never || a.n_nodes == 0) cur = kInvalid;
 				pend = kInvalid;
 				st.sp = 0;
-				if (SEEDED && a.n_nodes > 0) {
+				active = PASS == kAll || r.mine;
+				if (SEEDED && cur != kInvalid) {
 					// The lane starts at the best predicted cluster's entry instead of the root,
 					// which waits at the bottom of the stack; with several seeds the others sit
 					// above the root (the better on top) with their box entry distances. The
@@ -550,7 +626,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<N
 							if (q < a.n_seeds && sc[q] < a.n_clusters) {
 								const float *bx = a.cl_box + 6ull * sc[q];
 								const float lo[3] = {bx[0], bx[1], bx[2]}, hi[3] = {bx[3], bx[4], bx[5]};
-								const float tmin = child_slab(r, lo, hi, __builtin_inff());
+								const float tmin = child_slab(slab_ray(r), lo, hi, __builtin_inff());
 								const uint32_t ce = a.cl_entry[sc[q]];
 								if (ce != 0u && !__builtin_isnan(tmin)) {
 									sd[q] = ce;
@@ -569,6 +645,10 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<N
 						cur = sd[0];  // kInvalid: the next pop takes the best pushed cluster
 					}
 				}
+			}
+			if (PASS == kFast && !told && __ballot(!active && rank < avail) != 0ull) {
+				told = true;
+				if (lane == 0) __hip_atomic_store(flags + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 			}
 			const uint64_t took = n_need < avail ? n_need : avail;
 			chunk_next += took;
@@ -644,24 +724,23 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<N
 				const uint32_t tri = leaf_first(pend);
 				const uint32_t left = leaf_count(pend);
 				if (tri + left > a.n_tris) {  // corrupt entry: report, never read
-					atomicOr(a.counter + 8, 1u);
+					atomicOr(flags, 1u);
 					pend = kInvalid;
 					continue;
 				}
-				test_leaf<MODE == kWatertight>(a.tris, pend, r);  // the whole leaf (1..4 triangles)
+				test_leaf<MODE == kWatertight, PASS>(a.tris, pend, r);  // the whole leaf (1..4 triangles)
 				if (COUNT) c_tris += left;
 				pend = kInvalid;
 			}
 		} else if (cur != kInvalid && !(cur & kLeafBit)) {
 			if (cur >= a.n_nodes || st.sp + 7u > a.max_entries) {  // corrupt node or stack bound
-				atomicOr(a.counter + 8, 2u);
+				atomicOr(flags, 2u);
 				cur = kInvalid;
 				continue;
 			}
 			NodeHits h;
 			// the one-fma test's margins also cover the watertight mode's box corners
-			test_children<Node, NC, MODE == kWatertight>(nodes, a.nodes_q, cur, r, cull_limit(r, a),
-			                                             (MODE == kWatertight || a.cull) && r.fast, h);
+			ChildTest<Node, NC, MODE == kWatertight, PASS>::run(nodes, a.nodes_q, cur, r, cull_limit(r, a), h);
 			if (COUNT) ++c_nodes;
 			cur = h.key[0] != kMiss ? h.entry(h.key[0]) : kInvalid;
 			if (searched(cur)) cur = kInvalid;
@@ -677,12 +756,12 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<N
 		}
 	}
 	if (COUNT) {
-		atomicAdd(reinterpret_cast<unsigned long long *>(a.counter) + 1, c_nodes);
-		atomicAdd(reinterpret_cast<unsigned long long *>(a.counter) + 2, c_tris);
-		atomicAdd(reinterpret_cast<unsigned long long *>(a.counter) + 3, c_leaves);
-		atomicAdd(reinterpret_cast<unsigned long long *>(a.counter) + 5, c_nphase);
-		atomicAdd(reinterpret_cast<unsigned long long *>(a.counter) + 6, c_tphase);
-		atomicAdd(reinterpret_cast<unsigned long long *>(a.counter) + 7, c_culled);
+		atomicAdd(a.counter + C_NODES, c_nodes);
+		atomicAdd(a.counter + C_TRIS, c_tris);
+		atomicAdd(a.counter + C_LEAVES, c_leaves);
+		atomicAdd(a.counter + C_NPHASE, c_nphase);
+		atomicAdd(a.counter + C_TPHASE, c_tphase);
+		atomicAdd(a.counter + C_CULLED, c_culled);
 	}
 }
 
@@ -690,12 +769,24 @@ __global__ void k_zero(unsigned long long *p, int n) {
 	if (static_cast<int>(threadIdx.x) < n) p[threadIdx.x] = 0ull;
 }
 
+template <class Node, int S, int B, int MODE, bool NC, int PASS>
+void launch_pass(const KArgs &a, uint32_t grid, bool count, hipStream_t st) {
+	if (count)
+		hipLaunchKernelGGL((k_trace<Node, S, B, true, MODE, NC, PASS>), dim3(grid), dim3(B), 0, st, a);
+	else
+		hipLaunchKernelGGL((k_trace<Node, S, B, false, MODE, NC, PASS>), dim3(grid), dim3(B), 0, st, a);
+}
+
 template <class Node, int S, int B, int MODE, bool NC>
 void launch_nc(const KArgs &a, uint32_t grid, bool count, hipStream_t st) {
-	if (count)
-		hipLaunchKernelGGL((k_trace<Node, S, B, true, MODE, NC>), dim3(grid), dim3(B), 0, st, a);
-	else
-		hipLaunchKernelGGL((k_trace<Node, S, B, false, MODE, NC>), dim3(grid), dim3(B), 0, st, a);
+	if constexpr (std::is_same<Node, NodeF>::value) {
+		launch_pass<Node, S, B, MODE, NC, kAll>(a, grid, count, st);
+	} else {
+		launch_pass<Node, S, B, MODE, NC, kFast>(a, grid, count, st);
+		// seeds do not change a record: the second pass of the learned modes is the plain one
+		constexpr int REST = MODE == kSeeded || MODE == kSeededMulti ? kPlain : MODE;
+		launch_pass<Node, S, B, REST, NC, kRest>(a, grid, count, st);
+	}
 }
 
 // The batch always reads the never-cull masks (its builds are not read back); the other modes
@@ -786,10 +877,12 @@ hipError_t plan_trace(const Bvh8 &b, TraceScratch &s, const TraceParams &p, uint
 	return hipSuccess;
 }
 
-// Launches the traversal with the given counter (8 x u64, cleared here by a kernel) and spill
-// array (spill_depth entries per launched thread).
+// Launches the traversal with the given counters (clear: not all 0 yet, cleared here by a kernel)
+// and spill array (spill_depth entries per launched thread). `next`, when given, is cleared for
+// the launch that follows.
 hipError_t run_trace(const Bvh8 &b, const TraceParams &p, const float *rays, uint64_t n, uint32_t mask, void *out,
-                     hipStream_t st, uint32_t *counter, uint2 *spill, const TracePlan &pl, float *ms,
+                     hipStream_t st, unsigned long long *counter, bool clear, unsigned long long *next, uint2 *spill,
+                     const TracePlan &pl, float *ms,
                      TraceStats *stats, const SeedArgs *seeds, const BatchArgs *batch) {
 	const int B = p.block, S = p.lds_stack;
 	KArgs a;
@@ -800,6 +893,7 @@ hipError_t run_trace(const Bvh8 &b, const TraceParams &p, const float *rays, uin
 	a.rays = rays;
 	a.out = static_cast<uint8_t *>(out);
 	a.counter = counter;
+	a.next = next;
 	a.spill = spill;
 	a.n_rays = n;
 	a.n_nodes = b.n_nodes;
@@ -829,7 +923,7 @@ hipError_t run_trace(const Bvh8 &b, const TraceParams &p, const float *rays, uin
 	a.fast_scene = 1;
 	for (int k = 0; k < 6; ++k) a.fast_scene &= std::fabs(b.scene_box[k]) < 0x1p60f ? 1 : 0;
 
-	hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, st, reinterpret_cast<unsigned long long *>(a.counter), 8);
+	if (clear) hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, st, a.counter, static_cast<int>(kCounters));
 	hipEvent_t e0 = nullptr, e1 = nullptr;
 	if (ms) {
 		PRT_TRY(hipEventCreate(&e0));
@@ -848,16 +942,16 @@ hipError_t run_trace(const Bvh8 &b, const TraceParams &p, const float *rays, uin
 		(void)hipEventDestroy(e1);
 	}
 	if (stats) {
-		unsigned long long h[8];
+		unsigned long long h[kCounters];
 		PRT_TRY(hipMemcpyAsync(h, a.counter, sizeof(h), hipMemcpyDeviceToHost, st));
 		PRT_TRY(hipStreamSynchronize(st));
-		stats->node_visits = h[1];
-		stats->tri_tests = h[2];
-		stats->leaf_visits = h[3];
-		stats->errors = static_cast<uint32_t>(h[4]);
-		stats->node_phases = h[5];
-		stats->tri_phases = h[6];
-		stats->culled_pops = h[7];
+		stats->node_visits = h[C_NODES];
+		stats->tri_tests = h[C_TRIS];
+		stats->leaf_visits = h[C_LEAVES];
+		stats->errors = static_cast<uint32_t>(h[C_ERR]);
+		stats->node_phases = h[C_NPHASE];
+		stats->tri_phases = h[C_TPHASE];
+		stats->culled_pops = h[C_CULLED];
 	}
 	return hipSuccess;
 }
@@ -870,10 +964,31 @@ hipError_t trace_bvh8(const Bvh8 &b, TraceScratch &s, const TraceParams &p, cons
 	if (n == 0) return hipSuccess;
 	TracePlan pl;
 	PRT_TRY(plan_trace(b, s, p, n, pl));
-	PRT_TRY(s.counter.ensure(sizeof(unsigned long long) * 8));
+	static_assert(static_cast<int>(kCounters) <= TraceScratch::kSetWords, "counter set");
+	if (!s.counter.ptr) {
+		constexpr int words = TraceScratch::kSets * TraceScratch::kSetWords;
+		PRT_TRY(s.counter.ensure(sizeof(unsigned long long) * words));
+		hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, st, s.counter.as<unsigned long long>(), words);
+		s.clean = true;
+	}
 	PRT_TRY(s.spill.ensure(sizeof(uint2) * static_cast<uint64_t>(pl.spill_depth) * pl.grid * p.block));
-	return run_trace(b, p, rays, n, mask, out, st, s.counter.as<uint32_t>(), s.spill.as<uint2>(), pl, ms, stats, seeds,
-	                 batch);
+	// Sets 0 and 1 alternate: a launch clears the set of the next one, which saves that one its
+	// clearing kernel (1.3 to 4.3 us). A launch recorded into a graph may be
+	// replayed at any time: it has a set of its own and clears it itself.
+	hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+	PRT_TRY(hipStreamIsCapturing(st, &cap));
+	const bool captured = cap != hipStreamCaptureStatusNone;
+	const int set = captured ? 2 : s.next_set;
+	const bool clear = captured || !s.clean;
+	if (!captured) s.clean = false;
+	s.last_set = set;
+	PRT_TRY(run_trace(b, p, rays, n, mask, out, st, s.set(set), clear, captured ? nullptr : s.set(set ^ 1),
+	                  s.spill.as<uint2>(), pl, ms, stats, seeds, batch));
+	if (!captured) {
+		s.clean = true;
+		s.next_set = set ^ 1;
+	}
+	return hipSuccess;
 }
 
 // ------------------------------------------------------------ traversal without allocation
@@ -925,27 +1040,39 @@ hipError_t trace_bvh8_noalloc(const Bvh8 &b, TraceScratch &s, const TraceParams 
 	if (fit == 0) return hipErrorInvalidValue;
 	pl.grid = static_cast<uint32_t>(std::min<uint64_t>(pl.grid, fit));
 	uint8_t *base = static_cast<uint8_t *>(scratch_ptr);
-	return run_trace(b, p, rays, n, mask, out, st, reinterpret_cast<uint32_t *>(base),
+	return run_trace(b, p, rays, n, mask, out, st, reinterpret_cast<unsigned long long *>(base), true, nullptr,
 	                 reinterpret_cast<uint2 *>(base + kNoAllocCounterBytes), pl, nullptr, nullptr, nullptr, nullptr);
 }
 
-hipError_t trace_errors_at(TraceScratch &s, const uint32_t *counter, hipStream_t st, uint32_t *flags) {
+// ORs the error words of `sets` counter sets at `counter`.
+static hipError_t read_errors(TraceScratch &s, const unsigned long long *counter, int sets, hipStream_t st, uint32_t *flags) {
 	*flags = 0;
 	if (!counter) return hipSuccess;
+	const size_t bytes = sizeof(unsigned long long) * TraceScratch::kSetWords * sets;
 	if (!s.host_err) {
-		hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&s.host_err), sizeof(uint32_t));
+		hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&s.host_err),
+		                             sizeof(unsigned long long) * TraceScratch::kSetWords * TraceScratch::kSets);
 		if (e != hipSuccess) return e;
 	}
-	hipError_t e = hipMemcpyAsync(s.host_err, counter + 8, sizeof(uint32_t), hipMemcpyDeviceToHost, st);
+	hipError_t e = hipMemcpyAsync(s.host_err, counter, bytes, hipMemcpyDeviceToHost, st);
 	if (e == hipSuccess) e = hipStreamSynchronize(st);
-	if (e == hipSuccess) *flags = *s.host_err;
+	for (int k = 0; e == hipSuccess && k < sets; ++k)
+		*flags |= static_cast<uint32_t>(s.host_err[k * TraceScratch::kSetWords + C_ERR]);
 	return e;
+}
+
+hipError_t trace_errors_at(TraceScratch &s, const void *counter, hipStream_t st, uint32_t *flags) {
+	return read_errors(s, static_cast<const unsigned long long *>(counter), 1, st, flags);
 }
 
 #undef PRT_TRY
 
 hipError_t trace_errors(TraceScratch &s, hipStream_t st, uint32_t *flags) {
-	return trace_errors_at(s, s.counter.ptr ? s.counter.as<uint32_t>() : nullptr, st, flags);
+	return read_errors(s, s.counter.as<unsigned long long>(), TraceScratch::kSets, st, flags);
+}
+
+const uint32_t *trace_error_word(const TraceScratch &s) {
+	return reinterpret_cast<const uint32_t *>(s.set(s.last_set) + C_ERR);
 }
 
 }  // namespace prt
