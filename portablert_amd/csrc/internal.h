@@ -143,9 +143,12 @@ struct TraceStats {
 	unsigned long long node_phases = 0, tri_phases = 0, culled_pops = 0;  // wave iterations
 };
 
+// Rays that the first pass of a traversal may list for the second (trace.hip).
+constexpr uint32_t kLeftMax = 4096;
+
 struct TraceScratch {
 	static constexpr int kSets = 3, kSetWords = 16;  // 0 and 1 alternate, 2 serves captured launches
-	DevBuf counter;  // kSets sets of work counter, statistics and error flags
+	DevBuf counter;  // kSets sets of work counter, statistics and error flags, and the list of kLeftMax rays
 	DevBuf spill;    // per-thread stack spill
 	int n_cus = 0;
 	int next_set = 0, last_set = 0;

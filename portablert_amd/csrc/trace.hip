@@ -35,6 +35,7 @@ struct KArgs {
 	const float *rays;
 	uint8_t *out;
 	unsigned long long *counter;  // kCounters words (C_*), all 0 at the start of the launch
+	unsigned long long *left;     // rays left to kRest: ray index | scene << 40, kLeftMax entries
 	unsigned long long *next;     // another set, cleared here for the launch that follows, or null
 	uint2 *spill;           // spill_depth entries per launched thread
 	uint64_t n_rays;
@@ -70,17 +71,19 @@ enum : int {
 	C_NODES = 1,      // statistics
 	C_TRIS = 2,
 	C_LEAVES = 3,
-	C_ERR = 4,        // low 32 bits: error flags, high 32 bits: 1 once a ray was left to the second pass
+	C_ERR = 4,        // low 32 bits: error flags, high 32 bits: rays left to the second pass (see kLeftMax)
 	C_NPHASE = 5,
 	C_TPHASE = 6,
 	C_CULLED = 7,
-	C_WORK_REST = 8,  // next ray (or tile) of the second pass
+	C_WORK_REST = 8,  // next ray (or tile, or list entry) of the second pass
 	kCounters = 9
 };
 
 // Quantized nodes are traversed in two launches: kFast takes the rays of the one-fma node test
-// and leaves the others (d_x = 0, magnitudes out of its range) to kRest, whose waves end at once
-// where there are none, else go through all rays again and take those. One kernel for both held
+// and leaves the others (d_x = 0, magnitudes out of its range) to kRest. Up to kLeftMax of them are
+// listed; past that kRest goes through all rays again and takes those (a second look at 24 M
+// rays in 382,000 tiles takes 4.8 ms, which a single such ray must not cost). With none its waves
+// end at once. One kernel for both held
 // the reference formula's registers against every ray: at the plain mode's 64 it spilled 10, and
 // with the treatment of d_x = 0 (child_slab) 58. kAll: fp32 nodes, one node test for every ray.
 enum Pass : int { kAll = 0, kFast = 1, kRest = 2 };
@@ -522,9 +525,11 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<S
 	static_assert(std::is_same<Node, NodeF>::value == (PASS == kAll), "fp32 nodes take one pass");
 	unsigned long long *work = a.counter + (PASS == kRest ? C_WORK_REST : C_WORK);
 	uint32_t *flags = reinterpret_cast<uint32_t *>(a.counter + C_ERR);  // [0] errors, [1] rays left to kRest
-	if (PASS == kRest && flags[1] == 0u) return;
+	const uint32_t n_left = PASS == kRest ? flags[1] : 0u;
+	if (PASS == kRest && n_left == 0u) return;
+	const bool listed = PASS == kRest && n_left <= kLeftMax;
 	if (PASS != kRest && blockIdx.x == 0 && threadIdx.x < kCounters && a.next) a.next[threadIdx.x] = 0ull;
-	bool told = false;  // this wave has reported a ray left to kRest
+	bool told = false;  // the list is full: this wave adds nothing to it any more
 	constexpr bool MULTI = MODE == kSeededMulti, SEEDED = MODE == kSeeded || MULTI, BATCH = MODE == kBatch;
 	__shared__ uint2 lds[S * B];
 	const Node *nodes = static_cast<const Node *>(a.nodes);
@@ -562,7 +567,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<S
 		const uint64_t need = __ballot(!active);
 		const uint32_t n_need = __popcll(need);
 		if (n_need != 0u && !exhausted && (n_need >= a.refill || n_need == __popcll(__ballot(true)))) {
-			if (chunk_next >= chunk_end && BATCH) {
+			if (chunk_next >= chunk_end && BATCH && !listed) {
 				uint64_t tix = 0;
 				if (lane == 0) tix = atomicAdd(work, 1ull);
 				tix = uniform64(tix);
@@ -581,8 +586,9 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<S
 				if (lane == 0) base = atomicAdd(work, static_cast<unsigned long long>(a.chunk));
 				base = uniform64(base);
 				chunk_next = base;
-				chunk_end = base + a.chunk < a.n_rays ? base + a.chunk : a.n_rays;
-				if (base >= a.n_rays) {
+				const uint64_t n_work = listed ? n_left : a.n_rays;
+				chunk_end = base + a.chunk < n_work ? base + a.chunk : n_work;
+				if (base >= n_work) {
 					exhausted = true;
 					__builtin_amdgcn_s_setprio(0);
 				}
@@ -593,10 +599,16 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<S
 			                                                __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(need), 0u));
 			if (!active && rank < avail) {
 				ray_idx = chunk_next + rank;
+				uint32_t scene = chunk_scene;
+				if (listed) {
+					const unsigned long long e = a.left[ray_idx];
+					ray_idx = e & ((1ull << 40) - 1ull);
+					scene = static_cast<uint32_t>(e >> 40);
+				}
 				if (BATCH) {
-					const float2 si = a.scene_info[chunk_scene];
+					const float2 si = a.scene_info[scene];
 					load_ray<PASS, MODE == kWatertight>(a, ray_idx, si.x, si.y != 0.0f, r);
-					cur = chunk_scene;
+					cur = scene;
 				} else {
 					load_ray<PASS, MODE == kWatertight>(a, ray_idx, a.margin_abs, a.fast_scene != 0, r);
 					cur = 0u;
@@ -646,9 +658,20 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<S
 					}
 				}
 			}
-			if (PASS == kFast && !told && __ballot(!active && rank < avail) != 0ull) {
-				told = true;
-				if (lane == 0) __hip_atomic_store(flags + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+			if (PASS == kFast && !told) {
+				const uint64_t left = __ballot(!active && rank < avail);
+				if (left != 0ull) {
+					const uint32_t n = static_cast<uint32_t>(__popcll(left));
+					uint32_t at = 0;
+					if (lane == 0) at = atomicAdd(flags + 1, n);
+					at = __builtin_amdgcn_readfirstlane(at);
+					told = at + n > kLeftMax;
+					if (!active && rank < avail) {
+						const uint32_t k = at + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(left >> 32),
+						                                                  __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(left), 0u));
+						if (k < kLeftMax) a.left[k] = ray_idx | static_cast<unsigned long long>(BATCH ? chunk_scene : 0u) << 40;
+					}
+				}
 			}
 			const uint64_t took = n_need < avail ? n_need : avail;
 			chunk_next += took;
@@ -881,7 +904,8 @@ hipError_t plan_trace(const Bvh8 &b, TraceScratch &s, const TraceParams &p, uint
 // and spill array (spill_depth entries per launched thread). `next`, when given, is cleared for
 // the launch that follows.
 hipError_t run_trace(const Bvh8 &b, const TraceParams &p, const float *rays, uint64_t n, uint32_t mask, void *out,
-                     hipStream_t st, unsigned long long *counter, bool clear, unsigned long long *next, uint2 *spill,
+                     hipStream_t st, unsigned long long *counter, bool clear, unsigned long long *next,
+                     unsigned long long *left, uint2 *spill,
                      const TracePlan &pl, float *ms,
                      TraceStats *stats, const SeedArgs *seeds, const BatchArgs *batch) {
 	const int B = p.block, S = p.lds_stack;
@@ -894,6 +918,7 @@ hipError_t run_trace(const Bvh8 &b, const TraceParams &p, const float *rays, uin
 	a.out = static_cast<uint8_t *>(out);
 	a.counter = counter;
 	a.next = next;
+	a.left = left;
 	a.spill = spill;
 	a.n_rays = n;
 	a.n_nodes = b.n_nodes;
@@ -967,7 +992,7 @@ hipError_t trace_bvh8(const Bvh8 &b, TraceScratch &s, const TraceParams &p, cons
 	static_assert(static_cast<int>(kCounters) <= TraceScratch::kSetWords, "counter set");
 	if (!s.counter.ptr) {
 		constexpr int words = TraceScratch::kSets * TraceScratch::kSetWords;
-		PRT_TRY(s.counter.ensure(sizeof(unsigned long long) * words));
+		PRT_TRY(s.counter.ensure(sizeof(unsigned long long) * (words + kLeftMax)));
 		hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, st, s.counter.as<unsigned long long>(), words);
 		s.clean = true;
 	}
@@ -983,7 +1008,7 @@ hipError_t trace_bvh8(const Bvh8 &b, TraceScratch &s, const TraceParams &p, cons
 	if (!captured) s.clean = false;
 	s.last_set = set;
 	PRT_TRY(run_trace(b, p, rays, n, mask, out, st, s.set(set), clear, captured ? nullptr : s.set(set ^ 1),
-	                  s.spill.as<uint2>(), pl, ms, stats, seeds, batch));
+	                  s.set(TraceScratch::kSets), s.spill.as<uint2>(), pl, ms, stats, seeds, batch));
 	if (!captured) {
 		s.clean = true;
 		s.next_set = set ^ 1;
@@ -994,11 +1019,11 @@ hipError_t trace_bvh8(const Bvh8 &b, TraceScratch &s, const TraceParams &p, cons
 // ------------------------------------------------------------ traversal without allocation
 //
 // A device array of fixed size that the library never allocates or frees: the counter in its
-// first 256 bytes, the stack spill after it. Every GPU holds its own copy for the life of the
+// first 256 bytes, the stack spill after it, and the list of rays for the second pass. Every GPU holds its own copy for the life of the
 // process; its address on each device is looked up once (hipGetSymbolAddress, with that device
 // current) and only that address is passed to kernels or copies. All calls on one GPU share it:
 // calls that overlap on one GPU (other streams, other contexts) race.
-static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
+static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes + sizeof(unsigned long long) * kLeftMax];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -1041,6 +1066,7 @@ hipError_t trace_bvh8_noalloc(const Bvh8 &b, TraceScratch &s, const TraceParams 
 	pl.grid = static_cast<uint32_t>(std::min<uint64_t>(pl.grid, fit));
 	uint8_t *base = static_cast<uint8_t *>(scratch_ptr);
 	return run_trace(b, p, rays, n, mask, out, st, reinterpret_cast<unsigned long long *>(base), true, nullptr,
+	                 reinterpret_cast<unsigned long long *>(base + kNoAllocScratchBytes),
 	                 reinterpret_cast<uint2 *>(base + kNoAllocCounterBytes), pl, nullptr, nullptr, nullptr, nullptr);
 }
 

@@ -78,3 +78,26 @@ def test_orthographic_view_far_coordinates(gpu_ctx):
             rays[:, 3 + axis] = sign
             rays[::3, axis] = 1000.0
             assert_same(gpu_ctx.nearest_hits(rays, FULL), oracle.brute(tris, rays), what=f"axis {axis} {sign}")
+
+
+@pytest.mark.parametrize("n_rays", [900, 6000])
+def test_axis_rays_in_a_batch(gpu_ctx, n_rays):
+    """Rays of three scenes that the first pass leaves to the second: few enough to be listed, and
+    more than the list holds."""
+    import torch
+    rng = np.random.default_rng(n_rays)
+    tris = [grid_soup(rng, n, 4) for n in (300, 1, 700)]
+    rays = [axis_rays(rng, n) for n in (n_rays, 50, n_rays)]
+    d_tris, d_rays = (torch.from_numpy(np.concatenate(x)).cuda() for x in (tris, rays))
+    size, _ = prt.layout(FULL)
+    out = torch.zeros(sum(map(len, rays)) * size, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    batch = prt.Batch(gpu_ctx, list(map(len, tris)), list(map(len, rays)), FULL)
+    batch.capture(d_tris.data_ptr(), d_rays.data_ptr(), out.data_ptr())
+    want = one_nan(np.concatenate([oracle.brute(t, r) for t, r in zip(tris, rays)]))
+    for _ in range(3):  # every replay takes the second pass again
+        out.zero_()
+        torch.cuda.synchronize()
+        batch.replay()
+        batch.check()
+        assert_same(one_nan(out.cpu().numpy().view(prt.hit_dtype(FULL))), want, what=f"batch {n_rays}")
