@@ -246,10 +246,8 @@ int prt_mi355x_learned_train(prt_ctx *c, const float *d_rays, uint64_t n, int ep
 	for (int ep = 0; ep < epochs && e == hipSuccess; ++ep) {
 		for (uint64_t s = 0; s < steps && e == hipSuccess; ++s) {
 			const uint64_t first = s * batch;
-			e = mlp_encode(c->mlp, d_rays, first, batch, c->stream);
-			if (e == hipSuccess) e = mlp_forward_logits(c->mlp, batch, c->stream);
-			if (e == hipSuccess) e = mlp_backward(c->mlp, c->labels.as<uint32_t>() + first, batch, c->stream);
-			if (e == hipSuccess) e = mlp_adam(c->mlp, lr, c->stream);
+			e = mlp_forward_logits(c->mlp, d_rays, first, batch, c->stream);
+			if (e == hipSuccess) e = mlp_backward(c->mlp, c->labels.as<uint32_t>() + first, batch, lr, c->stream);
 		}
 	}
 	float loss = 0.0f;
@@ -382,9 +380,8 @@ int prt_mi355x_mlp_grad(prt_ctx *c, const float *rays, uint64_t n, const uint32_
 	if (e == hipSuccess) e = hipMemcpyAsync(dr.ptr, rays, n * 24, hipMemcpyHostToDevice, c->stream);
 	if (e == hipSuccess) e = hipMemcpyAsync(dl.ptr, labels, n * 4, hipMemcpyHostToDevice, c->stream);
 	const int rows = static_cast<int>(n);
-	if (e == hipSuccess) e = mlp_encode(c->mlp, dr.as<float>(), 0, rows, c->stream);
-	if (e == hipSuccess) e = mlp_forward_logits(c->mlp, rows, c->stream);
-	if (e == hipSuccess) e = mlp_backward(c->mlp, dl.as<uint32_t>(), rows, c->stream);
+	if (e == hipSuccess) e = mlp_forward_logits(c->mlp, dr.as<float>(), 0, rows, c->stream);
+	if (e == hipSuccess) e = mlp_backward(c->mlp, dl.as<uint32_t>(), rows, 0.0f, c->stream);
 	if (e == hipSuccess) e = hipMemcpyAsync(loss, c->mlp.loss.ptr, 4, hipMemcpyDeviceToHost, c->stream);
 	if (e == hipSuccess && x0) e = hipMemcpyAsync(x0, c->mlp.x0.ptr, n * kMlpIn * 2, hipMemcpyDeviceToHost, c->stream);
 	if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -418,8 +415,7 @@ int prt_mi355x_mlp_top4(prt_ctx *c, const float *rays, uint64_t n, uint32_t *top
 	if (e == hipSuccess) e = mlp_infer_top4(c->mlp, dr.as<float>(), 0, rows, dt.as<uint32_t>(), c->stream);
 	if (e == hipSuccess) e = hipMemcpyAsync(top4, dt.ptr, n * 16, hipMemcpyDeviceToHost, c->stream);
 	if (e == hipSuccess && logits) {
-		e = mlp_encode(c->mlp, dr.as<float>(), 0, rows, c->stream);
-		if (e == hipSuccess) e = mlp_forward_logits(c->mlp, rows, c->stream);
+		e = mlp_forward_logits(c->mlp, dr.as<float>(), 0, rows, c->stream);
 		if (e == hipSuccess)
 			e = hipMemcpy2DAsync(logits, kMlpOut * 4, c->mlp.logits.ptr, kMlpOutPad * 4, kMlpOut * 4, n,
 			                     hipMemcpyDeviceToHost, c->stream);

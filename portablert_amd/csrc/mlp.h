@@ -22,18 +22,17 @@ struct Mlp {
 	// parameters: fp32 master W^T [out][in] and bias, bf16 W^T and W, Adam moments, gradients
 	DevBuf w[4], b[4], wt_bf[4], w_bf[4], mw[4], vw[4], mb[4], vb[4], gw[4], gb[4];
 	// activations and work buffers (grown to the largest batch)
-	DevBuf x0, h[3], logits, dlog, dlog_t, dh[3], act_t, dact_t, split, loss;
+	DevBuf x0, h[3], logits, dlog, dlog_t, dh[3], act_t, dact_t, split, colsum, loss_row, loss;
 };
 
 hipError_t mlp_init(Mlp &m, uint64_t seed, hipStream_t st);
 hipError_t mlp_refresh_bf16(Mlp &m, hipStream_t st);
-// Encodes rays [first, first + rows) into m.x0.
-hipError_t mlp_encode(Mlp &m, const float *rays, uint64_t first, int rows, hipStream_t st);
-// x0 -> logits (fp32, m.logits [rows][kMlpOutPad]).
-hipError_t mlp_forward_logits(Mlp &m, int rows, hipStream_t st);
-// Softmax cross-entropy against labels, backward into m.gw / m.gb (rows multiple of 32).
-hipError_t mlp_backward(Mlp &m, const uint32_t *labels, int rows, hipStream_t st);
-hipError_t mlp_adam(Mlp &m, float lr, hipStream_t st);
+// Rays [first, first + rows) -> their encodings (m.x0), hidden layers and logits (fp32, m.logits
+// [rows][kMlpOutPad]).
+hipError_t mlp_forward_logits(Mlp &m, const float *rays, uint64_t first, int rows, hipStream_t st);
+// Softmax cross-entropy against labels, backward into m.gw / m.gb (rows multiple of 32) and, with
+// lr > 0, an Adam step.
+hipError_t mlp_backward(Mlp &m, const uint32_t *labels, int rows, float lr, hipStream_t st);
 // Encodes and runs rays [first, first + rows); writes the 4 best cluster logits' indices per
 // ray (descending, lower index first at equal logits) to top4 [rows][4].
 hipError_t mlp_infer_top4(Mlp &m, const float *rays, uint64_t first, int rows, uint32_t *top4, hipStream_t st);
