@@ -54,10 +54,13 @@ void apply_margin(prt_ctx *c) {
 	c->tp.margin_abs = std::ldexp(ext, -c->margin_log2 - 6);
 }
 
-int do_build(prt_ctx *c, uint64_t n) {
+// Builds from n device triangles.
+int do_build(prt_ctx *c, const float *tris, uint64_t n) {
 	bool bad = false;
 	double ms = 0.0;
-	hipError_t e = prt::build_bvh8(c->bs, n, c->bp, c->bvh, c->stream, &bad, &ms);
+	prt::SceneSet one;
+	one.tris = tris;
+	hipError_t e = prt::build_bvh8(c->bs, n, c->bp, c->bvh, c->stream, &bad, &ms, &one);
 	if (e != hipSuccess) {
 		c->has_scene = false;
 		return hip_fail(c, e, "BVH build");
@@ -71,6 +74,24 @@ int do_build(prt_ctx *c, uint64_t n) {
 	++c->scene_gen;
 	apply_margin(c);
 	return PRT_OK;
+}
+
+// Whether the kernels can read n triangles where the caller has them: 4-byte aligned and inside one
+// allocation of the context's GPU. Anything else is copied first, as hipMemcpyAsync takes it or
+// refuses it. (Builds and refits end before the call returns, so the caller's array outlives
+// them; the copy of 262,144 triangles took 5 us and a launch.)
+bool readable_in_place(const prt_ctx *c, const float *d_tris, uint64_t n) {
+	if (reinterpret_cast<uintptr_t>(d_tris) % 4) return false;
+	hipPointerAttribute_t at;
+	hipDeviceptr_t base = nullptr;
+	size_t size = 0;
+	if (hipPointerGetAttributes(&at, d_tris) != hipSuccess || at.type != hipMemoryTypeDevice || at.device != c->device ||
+	    hipMemGetAddressRange(&base, &size, const_cast<float *>(d_tris)) != hipSuccess) {
+		(void)hipGetLastError();
+		return false;
+	}
+	const uintptr_t at0 = reinterpret_cast<uintptr_t>(d_tris), b0 = reinterpret_cast<uintptr_t>(base);
+	return at0 >= b0 && at0 - b0 <= size && n <= (size - (at0 - b0)) / 36ull;
 }
 
 int over_limit(prt_ctx *c, uint64_t bytes, const char *what) {
@@ -149,6 +170,8 @@ void prt_mi355x_destroy(prt_ctx *c) {
 	                       &c->out_stage};
 	for (auto *b : bufs) b->release();
 	if (c->bs.host_misc) (void)hipHostFree(c->bs.host_misc);
+	for (hipEvent_t ev : c->bs.ev)
+		if (ev) (void)hipEventDestroy(ev);
 	c->pool.reset();
 	for (int b = 0; b < 2; ++b) {
 		if (c->pin_in[b]) (void)hipHostFree(c->pin_in[b]);
@@ -174,11 +197,11 @@ int prt_mi355x_device_name(const prt_ctx *c, char *buf, size_t cap) {
 	return PRT_OK;
 }
 
-// Refit from triangles already in c->bs.tri_in.
-static int do_refit(prt_ctx *c) {
+// Refit from device triangles.
+static int do_refit(prt_ctx *c, const float *tris) {
 	bool bad = false;
 	double ms = 0.0;
-	const hipError_t e = prt::refit_bvh8(c->bs, c->bvh, c->stream, &bad, &ms);
+	const hipError_t e = prt::refit_bvh8(c->bs, c->bvh, tris, c->stream, &bad, &ms);
 	if (e != hipSuccess) {
 		c->has_scene = false;
 		return hip_fail(c, e, "BVH refit");
@@ -203,10 +226,11 @@ static int refit_common(prt_ctx *c, const float *tris, uint64_t n, hipMemcpyKind
 	if (!tris) return fail(c, PRT_ERR_ARG, "refit: null triangle pointer");
 	if (hipSetDevice(c->device) != hipSuccess) return fail(c, PRT_ERR_HIP, "hipSetDevice");
 	hipError_t e = prt::wait_use(c);  // traversals on caller streams still read the old boxes
+	if (e == hipSuccess && kind == hipMemcpyDeviceToDevice && readable_in_place(c, tris, n)) return do_refit(c, tris);
 	if (e == hipSuccess) e = c->bs.tri_in.ensure(n * 36ull);
 	if (e == hipSuccess) e = hipMemcpyAsync(c->bs.tri_in.ptr, tris, n * 36ull, kind, c->stream);
 	if (e != hipSuccess) return hip_fail(c, e, "refit: triangle copy");
-	return do_refit(c);
+	return do_refit(c, c->bs.tri_in.as<float>());
 }
 
 int prt_mi355x_set_tris(prt_ctx *c, const float *tris, uint64_t n) {
@@ -222,7 +246,7 @@ int prt_mi355x_set_tris(prt_ctx *c, const float *tris, uint64_t n) {
 		e = hipMemcpyAsync(c->bs.tri_in.ptr, tris, n * 36ull, hipMemcpyHostToDevice, c->stream);
 		if (e != hipSuccess) return hip_fail(c, e, "set_tris: copy");
 	}
-	return do_build(c, n);
+	return do_build(c, c->bs.tri_in.as<float>(), n);
 }
 
 int prt_mi355x_refit(prt_ctx *c, const float *tris, uint64_t n) {
@@ -240,13 +264,14 @@ int prt_mi355x_set_tris_device(prt_ctx *c, const float *d_tris, uint64_t n) {
 	if (hipSetDevice(c->device) != hipSuccess) return fail(c, PRT_ERR_HIP, "hipSetDevice");
 	if (int r = over_limit(c, n * 36ull, "set_tris")) return r;
 	hipError_t e = prt::wait_use(c);  // traversals on caller streams still read the old BVH
+	if (e == hipSuccess && n && readable_in_place(c, d_tris, n)) return do_build(c, d_tris, n);
 	if (e == hipSuccess) e = c->bs.tri_in.ensure(std::max<uint64_t>(1, n) * 36ull);
 	if (e != hipSuccess) return hip_fail(c, e, "set_tris: triangle buffer");
 	if (n) {
 		e = hipMemcpyAsync(c->bs.tri_in.ptr, d_tris, n * 36ull, hipMemcpyDeviceToDevice, c->stream);
 		if (e != hipSuccess) return hip_fail(c, e, "set_tris: copy");
 	}
-	return do_build(c, n);
+	return do_build(c, c->bs.tri_in.as<float>(), n);
 }
 
 static int trace_common(prt_ctx *c, const float *d_rays, uint64_t n, uint32_t mask, void *d_out, hipStream_t st) {

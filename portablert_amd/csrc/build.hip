@@ -1743,92 +1743,152 @@ struct RefitArgs {
 	uint32_t *misc;
 };
 
-__global__ __launch_bounds__(kBlock) void k_refit_level(RefitArgs a, uint32_t begin, uint32_t end) {
-	for (uint32_t i = begin + blockIdx.x * kBlock + threadIdx.x; i < end; i += gridDim.x * kBlock) {
-		NodeF f = a.nf[i];
-		NodeQ q = a.nq[i];
-		float nlo[3] = {__builtin_inff(), __builtin_inff(), __builtin_inff()};
-		float nhi[3] = {-__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
-		uint32_t ncull = 0;  // never-cull mask from the moved triangles (cull_unsafe)
+// Node i with the 8 lanes of a group, one child slot a lane (one thread per node held a level for
+// 20 to 44 us: 8 children one after the other, each a dependent load, at two waves a SIMD). Every
+// lane of the wave takes part.
+__device__ __forceinline__ void refit_node(const RefitArgs &a, uint32_t i, bool on, CollapseLds &lds) {
+	const int g = static_cast<int>(threadIdx.x & 7u);
+	const uint32_t grp = (threadIdx.x >> 3) % kGroups;
+	uint4 head = make_uint4(0u, 0u, 0xFFFFFFFFu, 0xFFFFFFFFu);  // child_base, tri_base, meta
+	if (on) head = *reinterpret_cast<const uint4 *>(a.nf + i);
+	const uint32_t m = ((g < 4 ? head.z : head.w) >> (8 * (g & 3))) & 0xFFu;
+	float lo[3] = {__builtin_inff(), __builtin_inff(), __builtin_inff()};
+	float hi[3] = {-__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
+	bool flagged = false;  // the slot's subtree holds a triangle that is never culled (cull_unsafe)
+	if (meta_internal(m)) {
+		const uint32_t c = head.x + meta_offset(m);
+		if (c <= i || c >= a.n_nodes) {
+			atomicOr(a.misc + M_ERR, 2u);
+		} else {
+			const float4 cl = a.box[2ull * c], ch = a.box[2ull * c + 1];
+			lo[0] = cl.x; lo[1] = cl.y; lo[2] = cl.z;
+			hi[0] = ch.x; hi[1] = ch.y; hi[2] = ch.z;
+			flagged = __float_as_uint(ch.w) != 0u;
+		}
+	} else if (meta_used(m)) {
+		const uint32_t first = head.y + meta_offset(m), cnt = meta_count(m);
+		if (first + cnt > a.n_tris) {
+			atomicOr(a.misc + M_ERR, 2u);
+		} else {
+			for (uint32_t t = first; t < first + cnt; ++t) {
+				const uint4 *src = reinterpret_cast<const uint4 *>(a.tris + t);
+				const uint4 r0 = src[0], r1 = src[1], r2 = src[2];
+				const float v[9] = {__uint_as_float(r0.x), __uint_as_float(r0.y), __uint_as_float(r0.z),
+				                    __uint_as_float(r0.w), __uint_as_float(r1.x), __uint_as_float(r1.y),
+				                    __uint_as_float(r1.z), __uint_as_float(r1.w), __uint_as_float(r2.x)};
 #pragma unroll
-		for (int k = 0; k < 8; ++k) {
-			const uint32_t m = f.meta[k];
-			float lo[3] = {__builtin_inff(), __builtin_inff(), __builtin_inff()};
-			float hi[3] = {-__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
-			if (meta_internal(m)) {
-				const uint32_t c = f.child_base + meta_offset(m);
-				if (c <= i || c >= a.n_nodes) {
-					atomicOr(a.misc + M_ERR, 2u);
-				} else {
-					const float4 cl = a.box[2ull * c], ch = a.box[2ull * c + 1];
-					lo[0] = cl.x; lo[1] = cl.y; lo[2] = cl.z;
-					hi[0] = ch.x; hi[1] = ch.y; hi[2] = ch.z;
-					if (__float_as_uint(ch.w) != 0u) ncull |= 1u << k;
-				}
-			} else if (meta_used(m)) {
-				const uint32_t first = f.tri_base + meta_offset(m), cnt = meta_count(m);
-				if (first + cnt > a.n_tris) {
-					atomicOr(a.misc + M_ERR, 2u);
-				} else {
-					for (uint32_t t = first; t < first + cnt; ++t) {
-						for (int v = 0; v < 3; ++v)
+				for (int p = 0; p < 3; ++p)
 #pragma unroll
-							for (int ax = 0; ax < 3; ++ax) {
-								lo[ax] = fminf(lo[ax], a.tris[t].v[3 * v + ax]);
-								hi[ax] = fmaxf(hi[ax], a.tris[t].v[3 * v + ax]);
-							}
-						if (cull_unsafe(a.tris[t].v)) ncull |= 1u << k;
+					for (int ax = 0; ax < 3; ++ax) {
+						lo[ax] = fminf(lo[ax], v[3 * p + ax]);
+						hi[ax] = fmaxf(hi[ax], v[3 * p + ax]);
 					}
-				}
-			}
-#pragma unroll
-			for (int ax = 0; ax < 3; ++ax) {
-				f.lo[ax][k] = lo[ax];
-				f.hi[ax][k] = hi[ax];
-				nlo[ax] = fminf(nlo[ax], lo[ax]);
-				nhi[ax] = fmaxf(nhi[ax], hi[ax]);
+				flagged |= cull_unsafe(v);
 			}
 		}
-		a.box[2ull * i] = make_float4(nlo[0], nlo[1], nlo[2], 0.0f);
-		a.box[2ull * i + 1] = make_float4(nhi[0], nhi[1], nhi[2], __uint_as_float(ncull != 0u ? 1u : 0u));
-		q.ncull = static_cast<uint8_t>(ncull);
-		float sc[3];
-#pragma unroll
-		for (int ax = 0; ax < 3; ++ax) {
-			const int e = grid_exp(nlo[ax], nhi[ax]);
-			q.p[ax] = nlo[ax];
-			q.e[ax] = static_cast<int8_t>(e);
-			sc[ax] = exp2i(e);
-		}
-#pragma unroll
-		for (int k = 0; k < 8; ++k) {
-#pragma unroll
-			for (int ax = 0; ax < 3; ++ax) {
-				if (meta_used(f.meta[k])) {
-					quantize(f.lo[ax][k], f.hi[ax][k], nlo[ax], sc[ax], q.qlo[ax][k], q.qhi[ax][k]);
-				} else {
-					q.qlo[ax][k] = 255;
-					q.qhi[ax][k] = 0;
-				}
-			}
-		}
-		a.nf[i] = f;
-		a.nq[i] = q;
 	}
+	const uint32_t ncull = group_ballot(flagged);
+	NodeQ *q = reinterpret_cast<NodeQ *>(lds.q[grp]);
+	float *f = reinterpret_cast<float *>(lds.f[grp]);  // the node's boxes, lo then hi
+	float nlo[3], nhi[3];
+#pragma unroll
+	for (int ax = 0; ax < 3; ++ax) {
+		nlo[ax] = group_min(lo[ax]);
+		nhi[ax] = group_max(hi[ax]);
+		const int e = grid_exp(nlo[ax], nhi[ax]);
+		uint8_t ql = 255, qh = 0;
+		if (meta_used(m)) quantize(lo[ax], hi[ax], nlo[ax], exp2i(e), ql, qh);
+		q->qlo[ax][g] = ql;
+		q->qhi[ax][g] = qh;
+		f[8 * ax + g] = lo[ax];
+		f[24 + 8 * ax + g] = hi[ax];
+		if (g == 0) {
+			q->p[ax] = nlo[ax];
+			q->e[ax] = static_cast<int8_t>(e);
+		}
+	}
+	q->meta[g] = static_cast<uint8_t>(m);
+	if (g == 0) {
+		q->ncull = static_cast<uint8_t>(ncull);
+		q->child_base = head.x;
+		q->tri_base = head.y;
+	}
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+	if (on) {
+		if (g == 0) a.box[2ull * i] = make_float4(nlo[0], nlo[1], nlo[2], 0.0f);
+		if (g == 1) a.box[2ull * i + 1] = make_float4(nhi[0], nhi[1], nhi[2], __uint_as_float(ncull != 0u ? 1u : 0u));
+		uint4 *dq = reinterpret_cast<uint4 *>(a.nq + i), *df = reinterpret_cast<uint4 *>(a.nf + i) + 1;
+		constexpr int cq = sizeof(NodeQ) / 16, cf = sizeof(NodeF) / 16 - 1;
+		for (int k = g; k < cq + cf; k += 8) {
+			if (k < cq) dq[k] = lds.q[grp][k];
+			else df[k - cq] = lds.f[grp][k - cq];
+		}
+	}
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+}
+
+__global__ __launch_bounds__(kBlock) void k_refit_level(RefitArgs a, uint32_t begin, uint32_t end) {
+	__shared__ CollapseLds lds;
+	for (uint32_t i0 = begin + blockIdx.x * kGroups; i0 < end; i0 += gridDim.x * kGroups) {
+		const uint32_t i = i0 + (threadIdx.x >> 3);
+		refit_node(a, i, i < end, lds);
+	}
+}
+
+// Consecutive levels of at most kFewNodes nodes each, deepest first, by one workgroup: a launch for
+// each would take longer than its nodes.
+constexpr uint32_t kFewNodes = 256;
+constexpr int kFewLevels = 32;
+struct FewLevels {
+	int count;
+	uint32_t bound[kFewLevels + 1];  // level k of the run is [bound[k + 1], bound[k])
+};
+
+constexpr int kFewBlock = 1024;
+
+__global__ __launch_bounds__(kFewBlock) void k_refit_few(RefitArgs a, FewLevels f) {
+	__shared__ CollapseLds lds[kFewBlock / kBlock];
+	for (int k = 0; k < f.count; ++k) {
+		for (uint32_t i0 = f.bound[k + 1]; i0 < f.bound[k]; i0 += kFewBlock / 8) {
+			const uint32_t i = i0 + (threadIdx.x >> 3);
+			refit_node(a, i, i < f.bound[k], lds[threadIdx.x / kBlock]);
+		}
+		__syncthreads();  // the level's boxes are read by the next one
+	}
+	// the root's box goes back with the flags
+	if (f.bound[f.count] == 0u && threadIdx.x < 6u)
+		a.misc[M_SCENE + 6 + threadIdx.x] = f2o(reinterpret_cast<const float *>(a.box)[threadIdx.x + (threadIdx.x < 3u ? 0u : 1u)]);
 }
 
 }  // namespace
 
+// Host form of o2f.
+static float ordered_float(uint32_t u) {
+	union {
+		uint32_t u;
+		float f;
+	} c;
+	c.u = (u & 0x80000000u) ? (u & 0x7FFFFFFFu) : ~u;
+	return c.f;
+}
+
+// The scratch's pair of timing events, created at the first use.
+static hipError_t time_events(BuildScratch &s, hipEvent_t ev[2]) {
+	for (int k = 0; k < 2; ++k) {
+		if (!s.ev[k]) {
+			const hipError_t e = hipEventCreate(&s.ev[k]);
+			if (e != hipSuccess) return e;
+		}
+		ev[k] = s.ev[k];
+	}
+	return hipSuccess;
+}
+
 hipError_t build_bvh8(BuildScratch &s, uint64_t n64, const BuildParams &p, Bvh8 &out, hipStream_t st,
                       bool *bad_input, double *build_ms, const SceneSet *scenes) {
-	auto h2f = [](uint32_t u) {
-		union {
-			uint32_t u;
-			float f;
-		} c;
-		c.u = (u & 0x80000000u) ? (u & 0x7FFFFFFFu) : ~u;
-		return c.f;
-	};
 #define PRT_TRY(x)                                                                                 \
 	do {                                                                                           \
 		hipError_t e_ = (x);                                                                       \
@@ -1875,11 +1935,10 @@ hipError_t build_bvh8(BuildScratch &s, uint64_t n64, const BuildParams &p, Bvh8 
 	PRT_TRY(out.nodes_f.ensure(sizeof(NodeF) * cap));
 	PRT_TRY(out.tris.ensure(sizeof(TriRec) * n));
 
-	hipEvent_t ev0 = nullptr, ev1 = nullptr;
+	hipEvent_t ev[2] = {nullptr, nullptr};
 	if (build_ms) {  // device time of the build kernels (allocations above are not counted)
-		PRT_TRY(hipEventCreate(&ev0));
-		PRT_TRY(hipEventCreate(&ev1));
-		PRT_TRY(hipEventRecord(ev0, st));
+		PRT_TRY(time_events(s, ev));
+		PRT_TRY(hipEventRecord(ev[0], st));
 	}
 	uint32_t *misc = s.misc.as<uint32_t>();
 	const float *tri_in = ss.tris ? ss.tris : s.tri_in.as<float>();
@@ -2061,7 +2120,7 @@ hipError_t build_bvh8(BuildScratch &s, uint64_t n64, const BuildParams &p, Bvh8 
 	emit();
 	if (ss.box) hipLaunchKernelGGL(k_scene_boxes, dim3(blocks_for(6ull * S)), dim3(kBlock), 0, st, misc, S, ss.box);
 	PRT_TRY(read_back());
-	if (build_ms) PRT_TRY(hipEventRecord(ev1, st));
+	if (build_ms) PRT_TRY(hipEventRecord(ev[1], st));
 	PRT_TRY(hipStreamSynchronize(st));
 	bool again = false;
 	if (!(hm[M_ERR] & 1u)) {
@@ -2086,22 +2145,20 @@ hipError_t build_bvh8(BuildScratch &s, uint64_t n64, const BuildParams &p, Bvh8 
 			hipLaunchKernelGGL(k_clear_err, dim3(1), dim3(64), 0, st, misc);
 			emit();
 			PRT_TRY(read_back());
-			if (build_ms) PRT_TRY(hipEventRecord(ev1, st));
+			if (build_ms) PRT_TRY(hipEventRecord(ev[1], st));
 			PRT_TRY(hipStreamSynchronize(st));
 			again = false;
 		}
 	}
 	if (build_ms) {
 		float ms = 0.0f;
-		PRT_TRY(hipEventElapsedTime(&ms, ev0, ev1));
+		PRT_TRY(hipEventElapsedTime(&ms, ev[0], ev[1]));
 		*build_ms = ms;
-		(void)hipEventDestroy(ev0);
-		(void)hipEventDestroy(ev1);
 	}
 	*bad_input = (hm[M_ERR] & 1u) != 0;
 	if (*bad_input) return hipSuccess;  // the caller reports the input; the tree is not used
 	if (hm[M_ERR] & 2u) return hipErrorUnknown;  // inconsistent build
-	for (int k = 0; k < 6; ++k) out.scene_box[k] = h2f(hm[M_SCENE + 6 + k]);
+	for (int k = 0; k < 6; ++k) out.scene_box[k] = ordered_float(hm[M_SCENE + 6 + k]);
 	uint32_t nodes = 0, placed = 0;
 	for (int l = 0; l < level && hm[M_LCNT + 2 * l]; ++l) {
 		if (hm[M_LBASE + l] != nodes) return hipErrorUnknown;
@@ -2117,7 +2174,7 @@ hipError_t build_bvh8(BuildScratch &s, uint64_t n64, const BuildParams &p, Bvh8 
 #undef PRT_TRY
 }
 
-hipError_t refit_bvh8(BuildScratch &s, Bvh8 &b, hipStream_t st, bool *bad_input, double *refit_ms) {
+hipError_t refit_bvh8(BuildScratch &s, Bvh8 &b, const float *tris, hipStream_t st, bool *bad_input, double *refit_ms) {
 #define PRT_TRY(x)                                                                                 \
 	do {                                                                                           \
 		hipError_t e_ = (x);                                                                       \
@@ -2126,49 +2183,18 @@ hipError_t refit_bvh8(BuildScratch &s, Bvh8 &b, hipStream_t st, bool *bad_input,
 	*bad_input = false;
 	const uint64_t n = b.n_tris;
 	if (n == 0 || b.n_nodes == 0) return hipSuccess;
-	if (b.levels.empty()) {
-		// level ranges from the node headers: level 0 is the root; the next level ends after the
-		// last internal child of the current one
-		std::vector<NodeF> h;
-		try {
-			h.resize(b.n_nodes);
-		} catch (...) {
-			return hipErrorOutOfMemory;
-		}
-		PRT_TRY(hipMemcpyAsync(h.data(), b.nodes_f.ptr, sizeof(NodeF) * b.n_nodes, hipMemcpyDeviceToHost, st));
-		PRT_TRY(hipStreamSynchronize(st));
-		uint32_t begin = 0, end = 1;
-		while (begin < end) {
-			b.levels.push_back(begin);
-			uint32_t next = end;
-			for (uint32_t i = begin; i < end; ++i)
-				for (int k = 0; k < 8; ++k)
-					if (meta_internal(h[i].meta[k]))
-						next = std::max(next, h[i].child_base + meta_offset(h[i].meta[k]) + 1u);
-			if (next > b.n_nodes) {
-				b.levels.clear();
-				return hipErrorUnknown;  // a child outside the tree
-			}
-			begin = end;
-			end = next;
-		}
-		if (begin != b.n_nodes) {
-			b.levels.clear();
-			return hipErrorUnknown;  // nodes not reachable level by level
-		}
-	}
+	if (b.levels.empty()) return hipErrorInvalidValue;  // the build leaves them
 	PRT_TRY(s.refit_box.ensure(sizeof(float4) * 2ull * b.n_nodes));
 	PRT_TRY(s.misc.ensure(sizeof(uint32_t) * misc_words(1)));
 	if (!s.host_misc) PRT_TRY(hipHostMalloc(&s.host_misc, sizeof(uint32_t) * misc_words(1)));
-	hipEvent_t ev0 = nullptr, ev1 = nullptr;
+	hipEvent_t ev[2] = {nullptr, nullptr};
 	if (refit_ms) {
-		PRT_TRY(hipEventCreate(&ev0));
-		PRT_TRY(hipEventCreate(&ev1));
-		PRT_TRY(hipEventRecord(ev0, st));
+		PRT_TRY(time_events(s, ev));
+		PRT_TRY(hipEventRecord(ev[0], st));
 	}
 	uint32_t *misc = s.misc.as<uint32_t>();
 	hipLaunchKernelGGL(k_init_misc, dim3(blocks_for(misc_words(1))), dim3(kBlock), 0, st, misc, misc_words(1));
-	hipLaunchKernelGGL(k_refit_tris, dim3(blocks_for(n)), dim3(kBlock), 0, st, s.tri_in.as<float>(), b.tris.as<TriRec>(),
+	hipLaunchKernelGGL(k_refit_tris, dim3(blocks_for(n)), dim3(kBlock), 0, st, tris, b.tris.as<TriRec>(),
 	                   static_cast<uint32_t>(n), misc);
 	RefitArgs ra;
 	ra.tris = b.tris.as<TriRec>();
@@ -2178,35 +2204,35 @@ hipError_t refit_bvh8(BuildScratch &s, Bvh8 &b, hipStream_t st, bool *bad_input,
 	ra.n_nodes = b.n_nodes;
 	ra.n_tris = static_cast<uint32_t>(n);
 	ra.misc = misc;
-	for (size_t l = b.levels.size(); l-- > 0;) {
-		const uint32_t begin = b.levels[l], end = l + 1 < b.levels.size() ? b.levels[l + 1] : b.n_nodes;
-		hipLaunchKernelGGL(k_refit_level, dim3(std::min<uint32_t>(blocks_for(end - begin), 2048)), dim3(kBlock), 0, st, ra,
+	auto level_end = [&](size_t l) { return l + 1 < b.levels.size() ? b.levels[l + 1] : b.n_nodes; };
+	for (size_t l = b.levels.size(); l > 0;) {  // levels l - 1, l - 2, ... are left
+		FewLevels few;
+		few.count = 0;
+		few.bound[0] = level_end(l - 1);
+		while (l > 0 && few.count < kFewLevels && level_end(l - 1) - b.levels[l - 1] <= kFewNodes) few.bound[++few.count] = b.levels[--l];
+		if (few.count) hipLaunchKernelGGL(k_refit_few, dim3(1), dim3(kFewBlock), 0, st, ra, few);
+		if (l == 0) break;
+		if (few.count == kFewLevels) continue;
+		--l;
+		const uint32_t begin = b.levels[l], end = level_end(l);
+		hipLaunchKernelGGL(k_refit_level, dim3(std::min<uint32_t>(blocks_for(end - begin, kGroups), 2048)), dim3(kBlock), 0, st, ra,
 		                   begin, end);
 	}
 	PRT_TRY(hipGetLastError());
-	if (refit_ms) PRT_TRY(hipEventRecord(ev1, st));
-	float4 root[2];
-	PRT_TRY(hipMemcpyAsync(root, ra.box, sizeof(root), hipMemcpyDeviceToHost, st));
+	if (refit_ms) PRT_TRY(hipEventRecord(ev[1], st));
 	PRT_TRY(hipMemcpyAsync(s.host_misc, misc, sizeof(uint32_t) * misc_words(1), hipMemcpyDeviceToHost, st));
 	PRT_TRY(hipStreamSynchronize(st));
 	if (refit_ms) {
 		float ms = 0.0f;
-		PRT_TRY(hipEventElapsedTime(&ms, ev0, ev1));
+		PRT_TRY(hipEventElapsedTime(&ms, ev[0], ev[1]));
 		*refit_ms = ms;
-		(void)hipEventDestroy(ev0);
-		(void)hipEventDestroy(ev1);
 	}
 	const uint32_t err = static_cast<const uint32_t *>(s.host_misc)[M_ERR];
 	*bad_input = (err & 1u) != 0;
 	if (*bad_input) return hipSuccess;  // the caller reports the input; the tree is not used
 	if (err & 2u) return hipErrorUnknown;
 	b.n_ncull = static_cast<const uint32_t *>(s.host_misc)[M_NCULL];
-	b.scene_box[0] = root[0].x;
-	b.scene_box[1] = root[0].y;
-	b.scene_box[2] = root[0].z;
-	b.scene_box[3] = root[1].x;
-	b.scene_box[4] = root[1].y;
-	b.scene_box[5] = root[1].z;
+	for (int k = 0; k < 6; ++k) b.scene_box[k] = ordered_float(static_cast<const uint32_t *>(s.host_misc)[M_SCENE + 6 + k]);
 	return hipSuccess;
 #undef PRT_TRY
 }

@@ -52,7 +52,7 @@ struct Bvh8 {
 	DevBuf nodes_q;          // NodeQ[n_nodes]
 	DevBuf nodes_f;          // NodeF[n_nodes]
 	DevBuf tris;             // TriRec[n_tris], in leaf order
-	std::vector<uint32_t> levels;  // first node of each BVH8 level (found at the first refit)
+	std::vector<uint32_t> levels;  // first node of each BVH8 level (not of a fixed-length build)
 };
 
 // Scratch of the LBVH build, kept across set_tris calls.
@@ -72,6 +72,7 @@ struct BuildScratch {
 	DevBuf refit_box;   // refit: float4[2 * n_nodes] node boxes
 	DevBuf cost;        // cost-optimal collapse: per-scene area scales, 8 floats per internal node
 	void *host_misc = nullptr;  // pinned mirror of the counters and scene 0's bounds
+	hipEvent_t ev[2] = {nullptr, nullptr};  // build and refit timing
 };
 
 struct BuildParams {
@@ -115,10 +116,10 @@ hipError_t build_bvh8(BuildScratch &s, uint64_t n, const BuildParams &p, Bvh8 &o
 // deeper than a fixed-length build allows. Synchronises st.
 hipError_t build_errors(BuildScratch &s, hipStream_t st, uint32_t *flags);
 
-// New vertex positions (s.tri_in, the same n triangles in input order) for the tree in `b`:
+// New vertex positions (device, the same n triangles in input order) for the tree in `b`:
 // leaf records and every node box are recomputed bottom-up, the topology is kept. Sets
 // *bad_input for a non-finite vertex (the tree is then not usable). Synchronises st.
-hipError_t refit_bvh8(BuildScratch &s, Bvh8 &b, hipStream_t st, bool *bad_input, double *refit_ms);
+hipError_t refit_bvh8(BuildScratch &s, Bvh8 &b, const float *tris, hipStream_t st, bool *bad_input, double *refit_ms);
 
 // Traversal tunables.
 struct TraceParams {

@@ -55,3 +55,6 @@ def test_slow_merging(gpu_ctx):
     gpu_ctx.set_tris(tris)
     check_bvh(gpu_ctx, tris)
     assert_same(gpu_ctx.nearest_hits(rays, FULL), oracle.brute(tris, rays), what="equal triangles")
+    gpu_ctx.refit(tris * np.float32(1.5))  # a level is one to a few nodes here, 80 levels deep
+    check_bvh(gpu_ctx, tris * np.float32(1.5))
+    assert_same(gpu_ctx.nearest_hits(rays, FULL), oracle.brute(tris * np.float32(1.5), rays), what="refit of a deep tree")
