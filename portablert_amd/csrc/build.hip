@@ -31,8 +31,10 @@ namespace prt {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kSortItems = 16;                       // keys per thread per radix tile
-constexpr int kSortTile = kBlock * kSortItems;       // 4096 keys per tile
+// Keys per thread of a radix tile (256, 1,024 or 4,096 keys): a tile's rounds are a serial chain, so
+// few keys take small tiles that use more CUs (262,144 keys in 64 tiles of 4,096 took 15.5 us a
+// scatter), many keys large ones (fewer counts to scan).
+inline int sort_items(uint64_t n) { return n <= 32768 ? 1 : n <= (2u << 20) ? 4 : 16; }
 constexpr uint32_t kNone = 0xFFFFFFFFu;
 constexpr int kMaxLevels = 128;                      // BVH8 levels of a build
 constexpr int kSceneShift = 30;                      // key = scene << 30 | 30-bit Morton code
@@ -234,12 +236,13 @@ __global__ __launch_bounds__(kBlock) void k_morton(const float4 *__restrict__ tb
 
 // ------------------------------------------------------------------------- radix sort
 
+template <int kSortItems>
 __global__ __launch_bounds__(kBlock) void k_hist(const uint64_t *__restrict__ keys, uint32_t n, int shift,
                                                  uint32_t *__restrict__ hist, uint32_t tiles) {
 	__shared__ uint32_t h[256];
 	h[threadIdx.x] = 0;
 	__syncthreads();
-	const uint64_t base = static_cast<uint64_t>(blockIdx.x) * kSortTile;
+	const uint64_t base = static_cast<uint64_t>(blockIdx.x) * kBlock * kSortItems;
 #pragma unroll 4
 	for (int r = 0; r < kSortItems; ++r) {
 		const uint64_t i = base + static_cast<uint64_t>(r) * kBlock + threadIdx.x;
@@ -253,8 +256,8 @@ constexpr int kScanItems = 16;                 // histogram entries per thread
 constexpr int kScanSeg = kBlock * kScanItems;  // entries per segment
 
 // Exclusive scan of hist (digit-major: entry d * tiles + t) in two levels: each segment of
-// 4096 entries is scanned in place by one workgroup and its total goes to seg[]; k_scan then
-// scans seg[] and the scatter adds seg[entry / 4096].
+// 4096 entries is scanned in place by one workgroup and its total goes to seg[]; the scatter scans
+// up to kBlock totals itself (k_scan more) and adds that of segment entry / 4096.
 __global__ __launch_bounds__(kBlock) void k_scan_seg(uint32_t *hist, uint32_t total, uint32_t *seg) {
 	__shared__ uint32_t part[kBlock];
 	const uint64_t base = static_cast<uint64_t>(blockIdx.x) * kScanSeg + static_cast<uint64_t>(threadIdx.x) * kScanItems;
@@ -312,22 +315,23 @@ __global__ __launch_bounds__(1024) void k_scan(uint32_t *hist, uint32_t total) {
 // consecutive threads write consecutive positions of a digit's run. The tile's count of a digit
 // is the difference of two consecutive entries of the scanned histogram: it is digit-major, so
 // the entry after a digit's last tile is the next digit's first.
+template <int kSortItems>
 __global__ __launch_bounds__(kBlock) void k_scatter(const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
                                                     uint64_t *__restrict__ kout, uint32_t *__restrict__ vout,
                                                     uint32_t n, int shift, const uint32_t *__restrict__ hist,
-                                                    const uint32_t *__restrict__ seg, uint32_t tiles) {
+                                                    const uint32_t *__restrict__ seg, uint32_t n_seg, uint32_t tiles) {
+	constexpr int kSortTile = kBlock * kSortItems;
 	__shared__ uint64_t skey[kSortTile];
 	__shared__ uint32_t sval[kSortTile];
 	__shared__ uint32_t run[256];                // next tile position of each digit
 	__shared__ uint32_t delta[256];              // output position minus tile position, per digit
+	__shared__ uint32_t wtot[kBlock / 64];
 	__shared__ uint8_t wcnt[kBlock / 64][256];  // keys of each digit in each wave of a round (<= 64)
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 	const uint32_t d = threadIdx.x;
 	const uint64_t total = 256ull * tiles;
 	const uint64_t e = static_cast<uint64_t>(d) * tiles + blockIdx.x;
-	const uint32_t g0 = hist[e] + seg[e / kScanSeg];
-	const uint32_t g1 = e + 1 < total ? hist[e + 1] + seg[(e + 1) / kScanSeg] : n;
-	const uint32_t cnt = g1 - g0;
+	const uint32_t h0 = hist[e], h1 = e + 1 < total ? hist[e + 1] : n;
 	const uint64_t base = static_cast<uint64_t>(blockIdx.x) * kSortTile;
 	uint64_t kk[kSortItems];
 	uint32_t vv[kSortItems];
@@ -337,16 +341,32 @@ __global__ __launch_bounds__(kBlock) void k_scatter(const uint64_t *__restrict__
 		kk[r] = i < n ? kin[i] : 0ull;
 		vv[r] = i < n ? vin[i] : 0u;
 	}
-	// exclusive scan of the tile's digit counts: each digit's first tile position
-	run[d] = cnt;
-	__syncthreads();
-	for (int sh = 1; sh < 256; sh <<= 1) {
-		const uint32_t a = d >= static_cast<uint32_t>(sh) ? run[d - sh] : 0u;
+	// inclusive scan over the workgroup's 256 threads
+	auto scan = [&](uint32_t v) {
+		for (int sh = 1; sh < 64; sh <<= 1) {
+			const uint32_t o = __shfl_up(v, sh);
+			if (lane >= sh) v += o;
+		}
+		if (lane == 63) wtot[wave] = v;
 		__syncthreads();
-		run[d] += a;
+		for (int w = 0; w < wave; ++w) v += wtot[w];
 		__syncthreads();
+		return v;
+	};
+	uint32_t s0 = 0, s1 = 0;  // what the segments before add to h0 and h1
+	if (n_seg <= static_cast<uint32_t>(kBlock)) {
+		const uint32_t v = d < n_seg ? seg[d] : 0u;
+		delta[d] = scan(v) - v;
+		__syncthreads();
+		s0 = delta[e / kScanSeg];
+		s1 = e + 1 < total ? delta[(e + 1) / kScanSeg] : 0u;
+	} else {
+		s0 = seg[e / kScanSeg];
+		s1 = e + 1 < total ? seg[(e + 1) / kScanSeg] : 0u;
 	}
-	const uint32_t lofs = run[d] - cnt;
+	const uint32_t g0 = h0 + s0, cnt = h1 + s1 - g0;
+	// exclusive scan of the tile's digit counts: each digit's first tile position
+	const uint32_t lofs = scan(cnt) - cnt;
 	run[d] = lofs;
 	delta[d] = g0 - lofs;
 	const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
@@ -1919,7 +1939,8 @@ hipError_t build_bvh8(BuildScratch &s, uint64_t n64, const BuildParams &p, Bvh8 
 		PRT_TRY(s.keys[k].ensure(sizeof(uint64_t) * n));
 		PRT_TRY(s.vals[k].ensure(sizeof(uint32_t) * n));
 	}
-	const uint32_t tiles = blocks_for(n, kSortTile);
+	const int items = sort_items(n);
+	const uint32_t tiles = blocks_for(n, kBlock * items);
 	const uint32_t hist_n = 256 * tiles, n_seg = blocks_for(hist_n, kScanSeg);
 	PRT_TRY(s.hist.ensure(sizeof(uint32_t) * (static_cast<uint64_t>(hist_n) + n_seg)));
 	PRT_TRY(s.bin.ensure(sizeof(uint4) * n + sizeof(uint32_t) * (nb + 2ull * n)));
@@ -1952,14 +1973,20 @@ hipError_t build_bvh8(BuildScratch &s, uint64_t n64, const BuildParams &p, Bvh8 
 	while (S > 1 && (1ull << (key_bits - kSceneShift)) < S) ++key_bits;
 	int cur = 0;
 	for (int shift = 0; shift < key_bits; shift += 8) {
-		hipLaunchKernelGGL(k_hist, dim3(tiles), dim3(kBlock), 0, st, s.keys[cur].as<uint64_t>(), n, shift,
-		                   s.hist.as<uint32_t>(), tiles);
-		uint32_t *seg = s.hist.as<uint32_t>() + hist_n;
-		hipLaunchKernelGGL(k_scan_seg, dim3(n_seg), dim3(kBlock), 0, st, s.hist.as<uint32_t>(), hist_n, seg);
-		hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, st, seg, n_seg);
-		hipLaunchKernelGGL(k_scatter, dim3(tiles), dim3(kBlock), 0, st, s.keys[cur].as<uint64_t>(),
-		                   s.vals[cur].as<uint32_t>(), s.keys[cur ^ 1].as<uint64_t>(), s.vals[cur ^ 1].as<uint32_t>(),
-		                   n, shift, s.hist.as<uint32_t>(), seg, tiles);
+		uint32_t *hist = s.hist.as<uint32_t>(), *seg = hist + hist_n;
+		const uint64_t *kin = s.keys[cur].as<uint64_t>();
+		uint64_t *kout = s.keys[cur ^ 1].as<uint64_t>();
+		const uint32_t *vin = s.vals[cur].as<uint32_t>();
+		uint32_t *vout = s.vals[cur ^ 1].as<uint32_t>();
+		const dim3 tg(tiles), tb(kBlock);
+		if (items == 1) hipLaunchKernelGGL(k_hist<1>, tg, tb, 0, st, kin, n, shift, hist, tiles);
+		else if (items == 4) hipLaunchKernelGGL(k_hist<4>, tg, tb, 0, st, kin, n, shift, hist, tiles);
+		else hipLaunchKernelGGL(k_hist<16>, tg, tb, 0, st, kin, n, shift, hist, tiles);
+		hipLaunchKernelGGL(k_scan_seg, dim3(n_seg), tb, 0, st, hist, hist_n, seg);
+		if (n_seg > static_cast<uint32_t>(kBlock)) hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, st, seg, n_seg);
+		if (items == 1) hipLaunchKernelGGL(k_scatter<1>, tg, tb, 0, st, kin, vin, kout, vout, n, shift, hist, seg, n_seg, tiles);
+		else if (items == 4) hipLaunchKernelGGL(k_scatter<4>, tg, tb, 0, st, kin, vin, kout, vout, n, shift, hist, seg, n_seg, tiles);
+		else hipLaunchKernelGGL(k_scatter<16>, tg, tb, 0, st, kin, vin, kout, vout, n, shift, hist, seg, n_seg, tiles);
 		cur ^= 1;
 	}
 	const uint64_t *keys = s.keys[cur].as<uint64_t>();
