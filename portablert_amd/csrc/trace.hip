@@ -47,6 +47,7 @@ struct KArgs {
 	uint32_t spill_depth;
 	uint32_t chunk;         // rays a wave reserves per atomic
 	uint32_t leaf_phase;    // triangle phase once parked lanes >= live lanes * leaf_phase / 64
+	uint32_t wide_grid;     // workgroups of k_trace_wide for the first pass, 0: k_trace
 	uint32_t refill;        // load new rays once at least this many lanes are idle (or all are)
 	float margin_rel;
 	float margin_abs;
@@ -788,6 +789,202 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<S
 	}
 }
 
+// -------------------------------------------------------------- eight lanes per ray, few rays
+//
+// A launch of few rays lasts as long as its slowest ray's chain of visits, and in k_trace a visit
+// is some 300 instructions of one lane after the node's loads (65,536 room rays: 138 us at one wave
+// per SIMD, most of it waiting). Here a group of 8 lanes traces a ray: a lane per child slot in the
+// node test, per triangle in a leaf. The children's order is a rank (7 lane exchanges instead of
+// the sorting network), all pushes are one LDS store, and near and far planes are picked by
+// address. A wave holds 8 rays, each traversed at its own pace: pop, node test and leaf test in
+// one iteration. Costs more issue slots per ray than k_trace, which takes larger launches. 65,536
+// rays: room 137 -> 102 us, 1.5 M-triangle soup 510 -> 325, icosphere camera 153 -> 90.
+constexpr int kWideStack = 32;   // LDS stack entries per ray; deeper ones in the spill array
+constexpr int kWidePad = 33;     // entry stride of a ray's stack (the groups' tops in different banks)
+constexpr int kWideBlock = 128;
+
+// Value of lane g ^ X of the group (X in 1..7).
+template <int X>
+__device__ __forceinline__ uint32_t xor_lane(uint32_t v) {
+	constexpr int quad = (X & 3) == 1 ? 0xB1 : (X & 3) == 2 ? 0x4E : 0x1B;  // lane ^ 1, ^ 2, ^ 3
+	if (X >= 4) v = __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, false);  // row_half_mirror: ^ 7
+	constexpr int rest = X >= 4 ? X ^ 7 : X;
+	constexpr int q = (rest & 3) == 1 ? 0xB1 : (rest & 3) == 2 ? 0x4E : 0x1B;
+	if (rest != 0) v = __builtin_amdgcn_update_dpp(0, v, X >= 4 ? q : quad, 0xF, 0xF, false);
+	return v;
+}
+
+struct WideHit {
+	float t, u, v;
+	uint32_t id;
+};
+
+template <int X>
+__device__ __forceinline__ void wide_best(WideHit &h) {
+	const float t = __uint_as_float(xor_lane<X>(__float_as_uint(h.t)));
+	const float u = __uint_as_float(xor_lane<X>(__float_as_uint(h.u)));
+	const float v = __uint_as_float(xor_lane<X>(__float_as_uint(h.v)));
+	const uint32_t id = xor_lane<X>(h.id);
+	if (better(t, id, h.t, h.id)) h = {t, u, v, id};
+}
+
+template <int MODE, bool NC>
+__global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_trace_wide(KArgs a) {
+	static_assert(MODE == kPlain || MODE == kWatertight, "one scene, no seeds");
+	__shared__ uint2 lds[kWideBlock / 8][kWidePad];
+	if (blockIdx.x == 0 && threadIdx.x < kCounters && a.next) a.next[threadIdx.x] = 0ull;
+	uint32_t *flags = reinterpret_cast<uint32_t *>(a.counter + C_ERR);  // [0] errors, [1] rays left to kRest
+	const uint8_t *nodes = static_cast<const uint8_t *>(a.nodes);
+	const uint32_t g = threadIdx.x & 7u, group = (blockIdx.x * kWideBlock + threadIdx.x) >> 3;
+	const uint32_t groups = gridDim.x * (kWideBlock / 8);
+	uint2 *stack = lds[threadIdx.x >> 3];
+	auto spilled = [&](uint32_t k) { return a.spill + (static_cast<uint64_t>(k - kWideStack) * groups + group); };
+	bool told = false;  // the list of left rays is full
+	Ray r;
+	uint32_t near_at[3] = {0, 0, 0};  // byte of this lane's near bound on each axis, in the node
+	uint64_t ray_idx = group;
+	bool active = false;
+	uint32_t cur = kInvalid, sp = 0;
+	for (;;) {
+		const bool full = __ballot(told) != 0ull;  // the same in every lane
+		// ---- a group without a ray takes its next one
+		if (!active && ray_idx < a.n_rays) {
+			load_ray<kFast, MODE == kWatertight>(a, ray_idx, a.margin_abs, a.fast_scene != 0, r);
+			active = r.mine;
+			const uint64_t left = __ballot(!active && g == 0u);
+			if (left != 0ull && !full) {  // to the second pass: one atomic for the wave's groups
+				const uint32_t lane = threadIdx.x & 63u, n = static_cast<uint32_t>(__popcll(left));
+				const uint32_t lead = static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(left))) - 1u;
+				uint32_t at = 0;
+				if (lane == lead) {
+					at = __hip_atomic_load(flags + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+					if (at <= kLeftMax) at = atomicAdd(flags + 1, n);
+				}
+				at = __builtin_amdgcn_readlane(at, lead);
+				told = at + n > kLeftMax;
+				const uint32_t k = at + static_cast<uint32_t>(__popcll(left & ((1ull << lane) - 1ull)));
+				if (!active && g == 0u && k < kLeftMax) a.left[k] = ray_idx;
+			}
+			if (!active) ray_idx += groups;
+			cur = r.never || a.n_nodes == 0 ? kInvalid : 0u;
+			sp = 0;
+#pragma unroll
+			for (int ax = 0; ax < 3; ++ax) near_at[ax] = 32u + 8u * ax + (r.inv[ax] >= 0.0f ? 0u : 24u) + g;
+		}
+		if (__ballot(active || ray_idx < a.n_rays) == 0ull) break;
+		if (!active) continue;
+		const float limit = cull_limit(r, a);
+		// ---- next entry: the nearest child of the last node, else the stack's top (culled again)
+		if (cur == kInvalid) {
+			const uint32_t klim = key_limit(limit);
+			while (cur == kInvalid && sp > 0) {
+				--sp;
+				const uint2 e = sp < static_cast<uint32_t>(kWideStack) ? stack[sp] : *spilled(sp);
+				if (e.y <= klim) cur = e.x;
+			}
+		}
+		if (cur == kInvalid) {  // ray finished
+			if (g == 0u) write_record(a, ray_idx, r);
+			active = false;
+			ray_idx += groups;
+			continue;
+		}
+		if (!(cur & kLeafBit)) {
+			if (cur >= a.n_nodes || sp + 7u > a.max_entries) {  // corrupt node or stack bound
+				if (g == 0u) atomicOr(flags, 2u);
+				cur = kInvalid;
+				continue;
+			}
+			const uint8_t *node = nodes + static_cast<uint64_t>(cur) * sizeof(NodeQ);
+			const uint4 w0 = reinterpret_cast<const uint4 *>(node)[0], w1 = reinterpret_cast<const uint4 *>(node)[1];
+			uint32_t qn[3], qf[3];
+#pragma unroll
+			for (int ax = 0; ax < 3; ++ax) {
+				qn[ax] = node[near_at[ax]];
+				qf[ax] = node[r.inv[ax] >= 0.0f ? near_at[ax] + 24u : near_at[ax] - 24u];
+			}
+			const float p[3] = {__uint_as_float(w0.x), __uint_as_float(w0.y), __uint_as_float(w0.z)};
+			const uint32_t ncull = NC ? w0.w >> 24 : 0u;
+			float tn[3], tf[3];
+			// the one-fma bounds of ChildTest<NodeQ>, for this lane's child
+#pragma unroll
+			for (int ax = 0; ax < 3; ++ax) {
+				const float sc = exp2i(static_cast<int8_t>((w0.w >> (8 * ax)) & 0xFF));
+				const float step = sc * r.inv[ax];
+				const float base = (p[ax] - r.o[ax]) * r.inv[ax];
+				const float margin = (0x1p-18f * fabsf(r.inv[ax])) * fmaf(255.0f, sc, fabsf(p[ax]) + fabsf(r.o[ax]));
+				tn[ax] = fmaf(static_cast<float>(qn[ax]), step, base - margin);
+				tf[ax] = fmaf(static_cast<float>(qf[ax]), step, base + margin);
+			}
+			const float tmin = fmaxf(fmaxf(tn[0], tn[1]), tn[2]);
+			const float tmax = fminf(fminf(tf[0], tf[1]), tf[2]);
+			const float lim = ncull != 0u ? __builtin_inff() : limit;
+			const uint32_t meta = ((g < 4u ? w1.z : w1.w) >> (8u * (g & 3u))) & 0xFFu;
+			const bool hit = meta != kMetaEmpty && tmax >= 0.0f && tmin <= tmax && tmin <= lim;
+			uint32_t key = sort_key_finite(tmin, static_cast<int>(g));
+			if (NC && ((ncull >> g) & 1u)) key = kKeyNoCull | g;
+			if (!hit) key = kMiss;
+			// rank among the group's hits (keys differ in their slot bits)
+			uint32_t rank = 0;
+			rank += xor_lane<1>(key) < key;
+			rank += xor_lane<2>(key) < key;
+			rank += xor_lane<3>(key) < key;
+			rank += xor_lane<4>(key) < key;
+			rank += xor_lane<5>(key) < key;
+			rank += xor_lane<6>(key) < key;
+			rank += xor_lane<7>(key) < key;
+			uint32_t first = min(key, xor_lane<1>(key));
+			first = min(first, xor_lane<2>(first));
+			first = min(first, xor_lane<7>(first));
+			const uint32_t hits = static_cast<uint32_t>(__popcll((__ballot(hit) >> (threadIdx.x & 56u)) & 0xFFull));
+			const uint32_t lbase = leaf_base(w1.y);
+			// farthest lowest, so the nearest remaining child is on top
+			if (hit && rank != 0u) {
+				const uint32_t at = sp + hits - 1u - rank;
+				const uint2 e = make_uint2(child_entry(meta, w1.x, lbase), key);
+				if (at < static_cast<uint32_t>(kWideStack)) stack[at] = e;
+				else *spilled(at) = e;
+			}
+			sp += hits != 0u ? hits - 1u : 0u;
+			const uint32_t fs = first & 7u;
+			cur = first != kMiss ? child_entry(((fs < 4u ? w1.z : w1.w) >> (8u * (fs & 3u))) & 0xFFu, w1.x, lbase) : kInvalid;
+		}
+		if (cur != kInvalid && (cur & kLeafBit)) {
+			const uint32_t tri = leaf_first(cur), count = leaf_count(cur);
+			cur = kInvalid;
+			if (tri + count > a.n_tris) {  // corrupt entry: report, never read
+				if (g == 0u) atomicOr(flags, 1u);
+				continue;
+			}
+			// a lane per triangle (1..4), the best of them in every lane
+			WideHit h = {__builtin_inff(), 0.0f, 0.0f, kInvalid};
+			if (g < count) {
+				const uint4 *src = reinterpret_cast<const uint4 *>(a.tris + tri + g);
+				const uint4 x = src[0], y = src[1], z = src[2];
+				const float v[9] = {__uint_as_float(x.x), __uint_as_float(x.y), __uint_as_float(x.z),
+				                    __uint_as_float(x.w), __uint_as_float(y.x), __uint_as_float(y.y),
+				                    __uint_as_float(y.z), __uint_as_float(y.w), __uint_as_float(z.x)};
+				float inv[3];
+#pragma unroll
+				for (int k = 0; k < 3; ++k)
+					inv[k] = k > 0 && r.d[k] == 0.0f ? copysignf(__builtin_inff(), r.d[k]) : r.inv[k];
+				float t, u, vv;
+				const bool cand = MODE == kWatertight ? wt_candidate(v, r.o, r.d, inv, t, u, vv) : exact_candidate(v, r.o, r.d, inv, t, u, vv);
+				if (cand && better(t, z.y, h.t, h.id)) h = {t, u, vv, z.y};
+			}
+			wide_best<1>(h);
+			wide_best<2>(h);
+			wide_best<7>(h);
+			if (better(h.t, h.id, r.tb, r.idb)) {
+				r.tb = h.t;
+				r.ub = h.u;
+				r.vb = h.v;
+				r.idb = h.id;
+			}
+		}
+	}
+}
+
 __global__ void k_zero(unsigned long long *p, int n) {
 	if (static_cast<int>(threadIdx.x) < n) p[threadIdx.x] = 0ull;
 }
@@ -805,7 +1002,12 @@ void launch_nc(const KArgs &a, uint32_t grid, bool count, hipStream_t st) {
 	if constexpr (std::is_same<Node, NodeF>::value) {
 		launch_pass<Node, S, B, MODE, NC, kAll>(a, grid, count, st);
 	} else {
-		launch_pass<Node, S, B, MODE, NC, kFast>(a, grid, count, st);
+		if constexpr (MODE == kPlain || MODE == kWatertight) {
+			if (a.wide_grid) hipLaunchKernelGGL((k_trace_wide<MODE, NC>), dim3(a.wide_grid), dim3(kWideBlock), 0, st, a);
+			else launch_pass<Node, S, B, MODE, NC, kFast>(a, grid, count, st);
+		} else {
+			launch_pass<Node, S, B, MODE, NC, kFast>(a, grid, count, st);
+		}
 		// seeds do not change a record: the second pass of the learned modes is the plain one
 		constexpr int REST = MODE == kSeeded || MODE == kSeededMulti ? kPlain : MODE;
 		launch_pass<Node, S, B, REST, NC, kRest>(a, grid, count, st);
@@ -871,9 +1073,11 @@ struct TracePlan {
 	uint32_t max_entries = 0;  // stack bound 7 * depth + 8
 	uint32_t spill_depth = 0;  // stack entries per thread kept in global memory
 	uint32_t chunk = 64;       // rays a wave reserves at a time
+	uint32_t wide_grid = 0;    // workgroups of k_trace_wide, 0: k_trace
 };
 
-hipError_t plan_trace(const Bvh8 &b, TraceScratch &s, const TraceParams &p, uint64_t n, TracePlan &pl) {
+// several: seeds or scenes, which only k_trace takes.
+hipError_t plan_trace(const Bvh8 &b, TraceScratch &s, const TraceParams &p, uint64_t n, bool several, TracePlan &pl) {
 	if (s.n_cus == 0) {
 		int dev = 0;
 		PRT_TRY(hipGetDevice(&dev));
@@ -899,10 +1103,26 @@ hipError_t plan_trace(const Bvh8 &b, TraceScratch &s, const TraceParams &p, uint
 	const uint64_t need_threads = (n + 63) / 64 * 64;
 	grid64 = std::max<uint64_t>(1, std::min<uint64_t>(grid64, (need_threads + B - 1) / B));
 	pl.grid = static_cast<uint32_t>(grid64);
+	// Eight lanes per ray while the rays take at most one and a half rounds of the chip's 65,536
+	// groups (one for the watertight test, which culls nothing). One lane against eight, in us, for
+	// room, 1.5 M-triangle soup and icosphere camera: 16,384 rays 121 / 63, 506 / 287, 127 / 76; 98,304
+	// rays 160 / 135, 519 / 369, 169 / 96; 131,072 rays 171 / 178, 535 / 555, 178 / 91. Watertight,
+	// 65,536 rays: 358 / 300, 1344 / 1211, 231 / 169; 131,072 rays 396 / 484, 1393 / 2021, 261 / 276.
+	const uint64_t resident = static_cast<uint64_t>(s.n_cus) * 32 * 8;
+	if (n <= (p.leaf_test == 1 ? resident : resident + resident / 2) && p.node_format != 0 && p.waves_per_cu <= 0 &&
+	    !p.count_stats && !several)
+		pl.wide_grid = static_cast<uint32_t>((std::min(n, resident) * 8 + kWideBlock - 1) / kWideBlock);
 	// stack bound: each visited node pushes at most 7 entries, so 7 * depth + 1 suffice
 	pl.max_entries = 7u * std::max(1u, b.depth) + 8u;
 	pl.spill_depth = pl.max_entries > static_cast<uint32_t>(S) ? pl.max_entries - S : 1u;
 	return hipSuccess;
+}
+
+// Spill entries of either kernel of the first pass (k_trace's also serve the second).
+uint64_t spill_entries(const TracePlan &pl, const TraceParams &p) {
+	const uint64_t one = static_cast<uint64_t>(pl.spill_depth) * pl.grid * p.block;
+	const uint64_t deep = pl.max_entries > static_cast<uint32_t>(kWideStack) ? pl.max_entries - kWideStack : 0u;
+	return std::max(one, deep * pl.wide_grid * (kWideBlock / 8));
 }
 
 // Launches the traversal with the given counters (clear: not all 0 yet, cleared here by a kernel)
@@ -933,6 +1153,7 @@ hipError_t run_trace(const Bvh8 &b, const TraceParams &p, const float *rays, uin
 	a.mask = mask;
 	a.spill_depth = pl.spill_depth;
 	a.chunk = pl.chunk;
+	a.wide_grid = pl.wide_grid;
 	a.leaf_phase = static_cast<uint32_t>(std::max(1, std::min(64, p.leaf_phase)));
 	a.refill = static_cast<uint32_t>(std::max(1, std::min(64, p.refill)));
 	a.margin_rel = p.margin_rel;
@@ -993,7 +1214,7 @@ hipError_t trace_bvh8(const Bvh8 &b, TraceScratch &s, const TraceParams &p, cons
                       const BatchArgs *batch) {
 	if (n == 0) return hipSuccess;
 	TracePlan pl;
-	PRT_TRY(plan_trace(b, s, p, n, pl));
+	PRT_TRY(plan_trace(b, s, p, n, seeds || batch, pl));
 	static_assert(static_cast<int>(kCounters) <= TraceScratch::kSetWords, "counter set");
 	if (!s.counter.ptr) {
 		constexpr int words = TraceScratch::kSets * TraceScratch::kSetWords;
@@ -1001,7 +1222,7 @@ hipError_t trace_bvh8(const Bvh8 &b, TraceScratch &s, const TraceParams &p, cons
 		hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, st, s.counter.as<unsigned long long>(), words);
 		s.clean = true;
 	}
-	PRT_TRY(s.spill.ensure(sizeof(uint2) * static_cast<uint64_t>(pl.spill_depth) * pl.grid * p.block));
+	PRT_TRY(s.spill.ensure(sizeof(uint2) * spill_entries(pl, p)));
 	// Sets 0 and 1 alternate: a launch clears the set of the next one, which saves that one its
 	// clearing kernel (1.3 to 4.3 us). A launch recorded into a graph may be
 	// replayed at any time: it has a set of its own and clears it itself.
@@ -1061,7 +1282,7 @@ hipError_t trace_bvh8_noalloc(const Bvh8 &b, TraceScratch &s, const TraceParams 
 	if (n == 0) return hipSuccess;
 	if (!scratch_ptr) return hipErrorInvalidValue;
 	TracePlan pl;
-	PRT_TRY(plan_trace(b, s, p, n, pl));
+	PRT_TRY(plan_trace(b, s, p, n, false, pl));
 	// as many workgroups as the spill part holds (the kernel is persistent: fewer waves trace
 	// the same rays)
 	const uint64_t per_group = sizeof(uint2) * static_cast<uint64_t>(pl.spill_depth) * p.block;
@@ -1069,6 +1290,7 @@ hipError_t trace_bvh8_noalloc(const Bvh8 &b, TraceScratch &s, const TraceParams 
 	*need_bytes = kNoAllocCounterBytes + per_group;
 	if (fit == 0) return hipErrorInvalidValue;
 	pl.grid = static_cast<uint32_t>(std::min<uint64_t>(pl.grid, fit));
+	if (sizeof(uint2) * spill_entries(pl, p) > kNoAllocScratchBytes - kNoAllocCounterBytes) pl.wide_grid = 0;
 	uint8_t *base = static_cast<uint8_t *>(scratch_ptr);
 	return run_trace(b, p, rays, n, mask, out, st, reinterpret_cast<unsigned long long *>(base), true, nullptr,
 	                 reinterpret_cast<unsigned long long *>(base + kNoAllocScratchBytes),
