@@ -206,6 +206,8 @@ int prt_mi355x_mlp_grad(prt_ctx *ctx, const float *rays6, uint64_t n, const uint
                         uint16_t *x0_bf16);
 int prt_mi355x_mlp_grads(prt_ctx *ctx, int layer, float *gw, float *gb);
 int prt_mi355x_mlp_top4(prt_ctx *ctx, const float *rays6, uint64_t n, uint32_t *top4, float *logits);
+// The best cluster of each ray, as the one-seed traversal computes it.
+int prt_mi355x_mlp_top1(prt_ctx *ctx, const float *rays6, uint64_t n, uint32_t *top1);
 
 /* ---- Batched multi-scene tracing. No counterpart in the reference, whose backends hold one
  * scene per set_tris and trace one ray vector per nearest_hits (backend.hpp:19-46): here many

@@ -329,6 +329,7 @@ def _bind_learned(L):
     L.prt_mi355x_mlp_grad.argtypes = [vp, vp, u64, vp, ctypes.POINTER(ctypes.c_float), vp]
     L.prt_mi355x_mlp_grads.argtypes = [vp, ci, vp, vp]
     L.prt_mi355x_mlp_top4.argtypes = [vp, vp, u64, vp, vp]
+    L.prt_mi355x_mlp_top1.argtypes = [vp, vp, u64, vp]
     L._learned_bound = True
     return L
 
@@ -404,6 +405,14 @@ def mlp_top4(ctx, rays, with_logits=False):
     ctx._check(_learned_lib().prt_mi355x_mlp_top4(ctx.h, _p(rays), n, _p(top),
                                                    _p(logits) if with_logits else None))
     return (top, logits) if with_logits else top
+
+
+def mlp_top1(ctx, rays):
+    """The best cluster of each host ray, as the one-seed traversal computes it."""
+    rays = np.ascontiguousarray(rays, dtype=np.float32).reshape(-1, 6)
+    top = np.empty(len(rays), np.uint32)
+    ctx._check(_learned_lib().prt_mi355x_mlp_top1(ctx.h, _p(rays), len(rays), _p(top)))
+    return top
 
 
 # ------------------------------------------------------------------ batched multi-scene tracing

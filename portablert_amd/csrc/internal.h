@@ -166,8 +166,8 @@ hipError_t trace_errors(TraceScratch &s, hipStream_t st, uint32_t *flags);
 // Traces n device rays against `b`, writing HitReg records at `out` (device) with the layout
 // of `mask`. Launches on `st`; does not synchronise. `ms` receives the duration of the
 // traversal kernel measured with HIP events when non-null (synchronises then).
-// Per-ray seed clusters for the learned traversal: 4 cluster ids per ray (>= count: none),
-// and each cluster's stack entry and fp32 box.
+// Per-ray seed clusters for the learned traversal: 4 cluster ids per ray, or one with
+// TraceParams::n_seeds == 1 (>= count: none), and each cluster's stack entry and fp32 box.
 struct SeedArgs {
 	const uint32_t *seeds;
 	const uint32_t *entry;

@@ -187,11 +187,13 @@ hipError_t make_labels(prt_ctx *c, const float *d_rays, uint64_t n, uint32_t *la
 
 constexpr uint64_t kInferChunk = 1u << 24;  // rays per inference launch: 8 Mi rays in one (1% faster than 1 Mi launches)
 
-hipError_t infer_all(prt_ctx *c, const float *d_rays, uint64_t n, hipStream_t st) {
-	PRT_TRY(c->top4.ensure(16 * std::max<uint64_t>(1, n)));
+// The `best` (1 or 4) most likely clusters of n device rays, to c->top4 [n][best].
+hipError_t infer_all(prt_ctx *c, const float *d_rays, uint64_t n, int best, hipStream_t st) {
+	PRT_TRY(c->top4.ensure(4 * best * std::max<uint64_t>(1, n)));
 	for (uint64_t f = 0; f < n; f += kInferChunk) {
 		const int rows = static_cast<int>(std::min<uint64_t>(kInferChunk, n - f));
-		PRT_TRY(mlp_infer_top4(c->mlp, d_rays, f, rows, c->top4.as<uint32_t>() + 4 * f, st));
+		uint32_t *out = c->top4.as<uint32_t>() + best * f;
+		PRT_TRY((best == 1 ? mlp_infer_top1 : mlp_infer_top4)(c->mlp, d_rays, f, rows, out, st));
 	}
 	return hipSuccess;
 }
@@ -286,7 +288,7 @@ int prt_mi355x_nearest_hits_learned_device(prt_ctx *c, const float *d_rays, uint
 		if (e == hipSuccess) e = hipEventCreate(&e2);
 		if (e == hipSuccess) e = hipEventRecord(e0, st);
 	}
-	if (e == hipSuccess) e = infer_all(c, d_rays, n, st);
+	if (e == hipSuccess) e = infer_all(c, d_rays, n, c->tp.n_seeds > 1 ? 4 : 1, st);
 	if (e == hipSuccess && c->time_kernel) e = hipEventRecord(e1, st);
 	SeedArgs sa{c->top4.as<uint32_t>(), c->clusters.entry.as<uint32_t>(), c->clusters.box.as<float>(), c->clusters.count};
 	prt::TraceStats stats;
@@ -317,7 +319,7 @@ int prt_mi355x_learned_eval(prt_ctx *c, const float *d_rays, uint64_t n, double 
 	if (!d_rays || n == 0) return fail(c, PRT_ERR_ARG, "learned_eval: no rays");
 	hipError_t e = c->labels.ensure(4 * n);
 	if (e == hipSuccess) e = make_labels(c, d_rays, n, c->labels.as<uint32_t>());
-	if (e == hipSuccess) e = infer_all(c, d_rays, n, c->stream);
+	if (e == hipSuccess) e = infer_all(c, d_rays, n, 4, c->stream);
 	DevBuf cnt;
 	if (e == hipSuccess) e = cnt.ensure(16);
 	if (e == hipSuccess) e = hipMemsetAsync(cnt.ptr, 0, 16, c->stream);
@@ -424,6 +426,20 @@ int prt_mi355x_mlp_top4(prt_ctx *c, const float *rays, uint64_t n, uint32_t *top
 	dr.release();
 	dt.release();
 	return e == hipSuccess ? PRT_OK : hip_fail(c, e, "mlp_top4");
+}
+
+// The same for the best cluster alone, by the inference of the one-seed traversal.
+int prt_mi355x_mlp_top1(prt_ctx *c, const float *rays, uint64_t n, uint32_t *top1) {
+	if (!c || !rays || !top1 || n == 0 || n > 65536) return PRT_ERR_ARG;
+	if (int r = check_learned(c)) return r;
+	DevBuf dr, dt;
+	hipError_t e = dr.ensure(n * 24);
+	if (e == hipSuccess) e = dt.ensure(n * 4);
+	if (e == hipSuccess) e = hipMemcpyAsync(dr.ptr, rays, n * 24, hipMemcpyHostToDevice, c->stream);
+	if (e == hipSuccess) e = mlp_infer_top1(c->mlp, dr.as<float>(), 0, static_cast<int>(n), dt.as<uint32_t>(), c->stream);
+	if (e == hipSuccess) e = hipMemcpyAsync(top1, dt.ptr, n * 4, hipMemcpyDeviceToHost, c->stream);
+	if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+	return e == hipSuccess ? PRT_OK : hip_fail(c, e, "mlp_top1");
 }
 
 }  // extern "C"

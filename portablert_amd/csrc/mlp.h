@@ -19,8 +19,9 @@ struct Mlp {
 	bool ready = false;
 	int step = 0;
 	float scene_lo[3] = {0, 0, 0}, scene_inv_ext[3] = {1, 1, 1};
-	// parameters: fp32 master W^T [out][in] and bias, bf16 W^T and W, Adam moments, gradients
-	DevBuf w[4], b[4], wt_bf[4], w_bf[4], mw[4], vw[4], mb[4], vb[4], gw[4], gb[4];
+	// parameters: fp32 master W^T [out][in] and bias, bf16 W^T, W and W^T in MFMA
+	// fragment order, Adam moments, gradients
+	DevBuf w[4], b[4], wt_bf[4], w_bf[4], wt_frag[4], mw[4], vw[4], mb[4], vb[4], gw[4], gb[4];
 	// activations and work buffers (grown to the largest batch)
 	DevBuf x0, h[3], logits, dlog, dlog_t, dh[3], act_t, dact_t, split, colsum, loss_row, loss;
 };
@@ -36,6 +37,8 @@ hipError_t mlp_backward(Mlp &m, const uint32_t *labels, int rows, float lr, hipS
 // Encodes and runs rays [first, first + rows); writes the 4 best cluster logits' indices per
 // ray (descending, lower index first at equal logits) to top4 [rows][4].
 hipError_t mlp_infer_top4(Mlp &m, const float *rays, uint64_t first, int rows, uint32_t *top4, hipStream_t st);
+// The same for the best cluster only, to top1 [rows].
+hipError_t mlp_infer_top1(Mlp &m, const float *rays, uint64_t first, int rows, uint32_t *top1, hipStream_t st);
 
 // Clusters of a BVH8: up to kClusters subtrees that partition the triangles.
 struct Clusters {

@@ -42,6 +42,12 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
 }
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float(static_cast<uint32_t>(h) << 16); }
 
+// Place of weight (row, col) of a W^T [rows][cols] in its fragment order: 16 rows x 32 columns follow
+// each other as the MFMA operand of 64 lanes x 8 values, so a wave loads a fragment as 1 KB in a row.
+__device__ __forceinline__ size_t fragment_at(int row, int col, int cols) {
+	return (static_cast<size_t>(row >> 4) * (cols >> 5) + (col >> 5)) * 512 + ((((col >> 3) & 3) << 4) | (row & 15)) * 8 + (col & 7);
+}
+
 enum Epi : int {
 	E_BIAS_F32 = 0,   // out f32 = acc + bias[n]
 	E_MASK_BF16 = 1,  // out bf16 = acc * (aux_bf16[m][n] > 0)
@@ -227,9 +233,9 @@ struct FusedArgs {
 	uint64_t first;
 	int rows;
 	float4 lo, inv_ext;
-	const uint16_t *w[4];  // W^T bf16 [out][in]
+	const uint16_t *w[4];  // W^T bf16 [out][in]; in fragment order for k_mlp_top1
 	const float *b[4];
-	uint32_t *top4;        // [rows][4]
+	uint32_t *seeds;       // [rows][4] (k_mlp_top4) or [rows] (k_mlp_top1)
 };
 
 // One hidden layer computed per wave, without barriers between its tiles: every wave loads all 64
@@ -296,19 +302,22 @@ __device__ __forceinline__ void hidden_layer_pw(uint16_t *X, uint16_t *W, const 
 	__syncthreads();
 }
 
-// The encodings of rays r0..r0+63 in X; rows past the end are zero. Four threads per ray: inputs
-// 0-2 or 3-5, frequencies 0-7 or 8-15.
+// The encodings of rays r0..r0+ROWS-1 in X; rows past the end are zero. A quarter of a ray at a time:
+// inputs 0-2 or 3-5, frequencies 0-7 or 8-15.
+template <int ROWS>
 __device__ __forceinline__ void encode_rows(const FusedArgs &a, int r0, uint16_t *X) {
-	const int tid = threadIdx.x, row = tid >> 2, half = (tid >> 1) & 1, fq = tid & 1;
-	uint16_t *o = X + row * kFStride;
-	if (r0 + row < a.rows) {
-		encode_quarter(a.rays + 6 * (a.first + r0 + row), a.lo, a.inv_ext, half * 3, fq * 8, o);
-	} else {
-		uint32_t *o32 = reinterpret_cast<uint32_t *>(o);
+	for (int task = threadIdx.x; task < ROWS * 4; task += 256) {
+		const int row = task >> 2, half = (task >> 1) & 1, fq = task & 1;
+		uint16_t *o = X + row * kFStride;
+		if (r0 + row < a.rows) {
+			encode_quarter(a.rays + 6 * (a.first + r0 + row), a.lo, a.inv_ext, half * 3, fq * 8, o);
+		} else {
+			uint32_t *o32 = reinterpret_cast<uint32_t *>(o);
 #pragma unroll
-		for (int q = 0; q < 3; ++q)
+			for (int q = 0; q < 3; ++q)
 #pragma unroll
-			for (int jj = 0; jj < 8; ++jj) o32[(half * 3 + q) * 16 + fq * 8 + jj] = 0u;
+				for (int jj = 0; jj < 8; ++jj) o32[(half * 3 + q) * 16 + fq * 8 + jj] = 0u;
+		}
 	}
 }
 
@@ -330,7 +339,7 @@ __global__ __launch_bounds__(256, 2) void k_hidden(FusedArgs a, HiddenOut out) {
 				*reinterpret_cast<u32x4 *>(dst + static_cast<size_t>(r0 + r) * cols + c) = *reinterpret_cast<const u32x4 *>(X + r * kFStride + c);
 		}
 	};
-	encode_rows(a, r0, X);
+	encode_rows<kFRows>(a, r0, X);
 	__syncthreads();
 	write(out.x0, kMlpIn);
 	hidden_layer_pw<kMlpIn>(X, W, a.w[0], a.b[0], lane, wave);
@@ -377,7 +386,7 @@ __global__ __launch_bounds__(256, 2) void k_mlp_top4(FusedArgs a) {
 	__shared__ __align__(16) uint16_t W[kFCols * kFStride];
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 	const int r0 = blockIdx.x * kFRows;
-	encode_rows(a, r0, X);
+	encode_rows<kFRows>(a, r0, X);
 	__syncthreads();
 	hidden_layer_pw<kMlpIn>(X, W, a.w[0], a.b[0], lane, wave);
 	hidden_layer_pw<kMlpHidden>(X, W, a.w[1], a.b[1], lane, wave);
@@ -568,7 +577,168 @@ __global__ __launch_bounds__(256, 2) void k_mlp_top4(FusedArgs a) {
 	top_merge(v, ix, 2);
 	if (opart == 0 && r0 + orow < a.rows) {
 		const uint32_t res[4] = {ix[0], ix[1], ix[2], ix[3]};
-		reinterpret_cast<uint4 *>(a.top4)[r0 + orow] = make_uint4(res[0], res[1], res[2], res[3]);
+		reinterpret_cast<uint4 *>(a.seeds)[r0 + orow] = make_uint4(res[0], res[1], res[2], res[3]);
+	}
+}
+
+// ------------------------------------------------------------- fused inference, the best cluster only
+//
+// One seed per ray is the traversal's default, and its argmax needs neither the logits' trip through
+// LDS nor the insertions of k_mlp_top4. A workgroup takes 64 rays, all of them as MFMA B operands
+// in every wave's registers; each wave owns 16 of a tile's 64 neurons and reads their weights from L2
+// straight into its A operands, a tile ahead, without LDS and without barriers. The results are the
+// transposed tile: a lane holds four neurons of one ray per 16 x 16 block and keeps that ray's best over
+// its neurons, four instructions an element, issued between the next tile's MFMAs. Each logit is the
+// same chain of products over K as in k_mlp_top4. 1 Mi rays: 1.93 ms (1.34 PFLOP/s) against 2.9 in
+// k_mlp_top4; 16,384 rays take 38 us. Bound by the weights' way from L2 (2.4 MB per 64 rays, 20 TB/s).
+constexpr int kRayTiles = 4, kTop1Rows = kRayTiles * 16;
+
+template <int K>
+__device__ __forceinline__ void load_rays(const uint16_t *X, int lane, bf16x8 (&xr)[kRayTiles][K / kBK]) {
+#pragma unroll
+	for (int i = 0; i < kRayTiles; ++i)
+#pragma unroll
+		for (int kk = 0; kk < K / kBK; ++kk)
+			xr[i][kk] = *reinterpret_cast<const bf16x8 *>(X + (i * 16 + (lane & 15)) * kFStride + kk * kBK + (lane >> 4) * 8);
+}
+
+template <int K>
+__device__ __forceinline__ void hidden_layer_t(uint16_t *X, const uint16_t *wt, const float *bias, int lane, int wave) {
+	constexpr int RT = kRayTiles, KS = K / kBK;
+	const int n0 = wave * 64;  // this wave's 64 neurons
+	const uint16_t *wsrc = wt + static_cast<size_t>(wave * 4 * KS) * 512 + lane * 8;
+	bf16x8 w[KS], xr[RT][KS];
+#pragma unroll
+	for (int kk = 0; kk < KS; ++kk) w[kk] = *reinterpret_cast<const bf16x8 *>(wsrc + kk * 512);
+	load_rays<K>(X, lane, xr);
+	__syncthreads();  // every wave holds X in registers: its space takes the outputs
+#pragma unroll
+	for (int t = 0; t < 4; ++t) {
+		f32x4 acc[RT];
+#pragma unroll
+		for (int i = 0; i < RT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+		const int n = n0 + t * 16 + (lane >> 4) * 4;
+		const f32x4 b = *reinterpret_cast<const f32x4 *>(bias + n);
+#pragma unroll
+		for (int kk = 0; kk < KS; ++kk) {
+#pragma unroll
+			for (int i = 0; i < RT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[kk], xr[i][kk], acc[i], 0, 0, 0);
+			if (t + 1 < 4) w[kk] = *reinterpret_cast<const bf16x8 *>(wsrc + ((t + 1) * KS + kk) * 512);
+		}
+#pragma unroll
+		for (int i = 0; i < RT; ++i) {
+			uint32_t h[4];
+#pragma unroll
+			for (int e = 0; e < 4; ++e) h[e] = f2bf(fmaxf(acc[i][e] + b[e], 0.0f));
+			*reinterpret_cast<uint2 *>(X + (i * 16 + (lane & 15)) * kFStride + n) = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+		}
+	}
+	__syncthreads();
+}
+
+__global__ __launch_bounds__(256, 2) void k_mlp_top1(FusedArgs a) {
+	constexpr int kRows = kTop1Rows, RT = kRayTiles, KS = kMlpHidden / kBK;
+	constexpr int kTiles = (kMlpOut + kFCols - 1) / kFCols;  // the last one holds the miss logit
+	static_assert(kTiles * kFCols <= kMlpOutPad && kTiles % 2 == 1, "padding rows are read; tiles go in pairs after the first");
+	__shared__ __align__(16) uint16_t X[kRows * kFStride];
+	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, quad = lane >> 4;
+	const int r0 = blockIdx.x * kRows;
+	encode_rows<kRows>(a, r0, X);
+	__syncthreads();
+	hidden_layer_t<kMlpIn>(X, a.w[0], a.b[0], lane, wave);
+	hidden_layer_t<kMlpHidden>(X, a.w[1], a.b[1], lane, wave);
+	hidden_layer_t<kMlpHidden>(X, a.w[2], a.b[2], lane, wave);
+	const uint16_t *wsrc = a.w[3] + wave * KS * 512 + lane * 8;
+	const float *bsrc = a.b[3] + wave * 16 + quad * 4;
+	bf16x8 w[KS], xr[RT][KS];
+#pragma unroll
+	for (int kk = 0; kk < KS; ++kk) w[kk] = *reinterpret_cast<const bf16x8 *>(wsrc + kk * 512);
+	load_rays<kMlpHidden>(X, lane, xr);
+	float best[RT];
+	uint32_t code[RT];  // tile * 4 + element
+#pragma unroll
+	for (int i = 0; i < RT; ++i) {
+		best[i] = -__builtin_inff();
+		code[i] = 0xFFFFFFFFu;
+	}
+	// a strict comparison keeps the lower neuron at equal logits
+	auto take = [&](int i, int e, float x, uint32_t c) {
+		const bool more = x > best[i];
+		best[i] = more ? x : best[i];
+		code[i] = more ? c + e : code[i];
+	};
+	// tile t's MFMAs into acc with the comparisons of tile t - 1's results (old, its bias ob) between
+	// them; each K step's weights of tile t + 1 are loaded once its own are used
+	auto step = [&](int t, f32x4 (&acc)[RT], f32x4 &b, const f32x4 (&old)[RT], const f32x4 &ob, bool first) {
+		const int next = t + 1 < kTiles ? t + 1 : t;
+		const uint16_t *ws = wsrc + static_cast<size_t>(next) * 4 * KS * 512;
+		b = *reinterpret_cast<const f32x4 *>(bsrc + t * kFCols);
+		const uint32_t c = static_cast<uint32_t>(t - 1) * 4u;
+#pragma unroll
+		for (int kk = 0; kk < KS; ++kk) {
+#pragma unroll
+			for (int i = 0; i < RT; ++i)
+				acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[kk], xr[i][kk], kk == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[i], 0, 0, 0);
+			w[kk] = *reinterpret_cast<const bf16x8 *>(ws + kk * 512);
+			if (!first) {
+#pragma unroll
+				for (int q = 0; q < RT / 2; ++q) {
+					const int at = kk * (RT / 2) + q;
+					take(at / 4, at % 4, old[at / 4][at % 4] + ob[at % 4], c);
+				}
+			}
+			__builtin_amdgcn_sched_barrier(0);
+		}
+	};
+	f32x4 acc0[RT], acc1[RT], b0, b1;
+	step(0, acc0, b0, acc1, b1, true);
+	for (int t = 1; t < kTiles; t += 2) {
+		step(t, acc1, b1, acc0, b0, false);
+		step(t + 1, acc0, b0, acc1, b1, false);
+	}
+#pragma unroll
+	for (int e = 0; e < 4; ++e) {  // the last tile's padding neurons are never taken
+		if ((kTiles - 1) * kFCols + wave * 16 + quad * 4 + e < kMlpOut) {
+#pragma unroll
+			for (int i = 0; i < RT; ++i) take(i, e, acc0[i][e] + b0[e], (kTiles - 1) * 4);
+		}
+	}
+	// the best of a ray's four lanes, then of the four waves
+	__syncthreads();
+	float *mv = reinterpret_cast<float *>(X);
+	uint32_t *mi = reinterpret_cast<uint32_t *>(X) + 4 * kRows;
+#pragma unroll
+	for (int i = 0; i < RT; ++i) {
+		float x = best[i];
+		uint32_t n = code[i] == 0xFFFFFFFFu ? code[i] : (code[i] >> 2) * kFCols + wave * 16 + quad * 4 + (code[i] & 3u);
+#pragma unroll
+		for (int m = 16; m < 64; m *= 2) {
+			const float ox = __shfl_xor(x, m);
+			const uint32_t on = __shfl_xor(n, m);
+			if (top_better(ox, on, x, n)) {
+				x = ox;
+				n = on;
+			}
+		}
+		if (quad == 0) {
+			mv[wave * kRows + i * 16 + lane] = x;
+			mi[wave * kRows + i * 16 + lane] = n;
+		}
+	}
+	__syncthreads();
+	if (tid < kRows && r0 + tid < a.rows) {
+		float x = mv[tid];
+		uint32_t n = mi[tid];
+#pragma unroll
+		for (int q = 1; q < 4; ++q) {
+			const float ox = mv[q * kRows + tid];
+			const uint32_t on = mi[q * kRows + tid];
+			if (top_better(ox, on, x, n)) {
+				x = ox;
+				n = on;
+			}
+		}
+		a.seeds[r0 + tid] = n;
 	}
 }
 
@@ -683,6 +853,7 @@ struct AdamPart {
 	const float *part;   // partial gradients [splits][n]
 	int splits;
 	uint16_t *bf, *bft;  // weights: bf16 copies W^T [rows][cols] and W [cols][rows]
+	uint16_t *frag;      // and W^T in fragment order
 	int rows, cols;      // bias: rows entries, of which the first cols are updated
 	unsigned first;      // first workgroup
 };
@@ -763,6 +934,7 @@ __global__ __launch_bounds__(256) void k_update(AdamArgs a) {
 			*reinterpret_cast<f32x4 *>(q.p + i) = p;
 			const uint32_t w0 = f2bf(p[0]) | static_cast<uint32_t>(f2bf(p[1])) << 16, w1 = f2bf(p[2]) | static_cast<uint32_t>(f2bf(p[3])) << 16;
 			*reinterpret_cast<uint2 *>(q.bf + i) = make_uint2(w0, w1);
+			*reinterpret_cast<uint2 *>(q.frag + fragment_at(r0 + r, c0 + c, q.cols)) = make_uint2(w0, w1);
 			reinterpret_cast<uint32_t *>(&t[r][c])[0] = w0;
 			reinterpret_cast<uint32_t *>(&t[r][c])[1] = w1;
 		}
@@ -797,11 +969,12 @@ __global__ __launch_bounds__(256) void k_fill_f32(float *p, size_t n, float v) {
 }
 
 __global__ __launch_bounds__(256) void k_to_bf16(const float *__restrict__ p, size_t n, uint16_t *__restrict__ bf,
-                                                 uint16_t *__restrict__ bft, int rows, int cols) {
+                                                 uint16_t *__restrict__ bft, uint16_t *__restrict__ frag, int rows, int cols) {
 	const size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
 	if (i >= n) return;
 	const uint16_t h = f2bf(p[i]);
 	bf[i] = h;
+	frag[fragment_at(static_cast<int>(i / cols), static_cast<int>(i % cols), cols)] = h;
 	if (bft) bft[static_cast<size_t>(i % cols) * rows + i / cols] = h;
 }
 
@@ -834,6 +1007,7 @@ hipError_t mlp_init(Mlp &m, uint64_t seed, hipStream_t st) {
 		PRT_TRY(m.w[l].ensure(n * 4));
 		PRT_TRY(m.b[l].ensure(kLayerOut[l] * 4));
 		PRT_TRY(m.wt_bf[l].ensure(n * 2));
+		PRT_TRY(m.wt_frag[l].ensure(n * 2));
 		PRT_TRY(m.w_bf[l].ensure(n * 2));
 		PRT_TRY(m.mw[l].ensure(n * 4));
 		PRT_TRY(m.vw[l].ensure(n * 4));
@@ -857,7 +1031,7 @@ hipError_t mlp_init(Mlp &m, uint64_t seed, hipStream_t st) {
 		hipLaunchKernelGGL(k_fill_f32, dim3(blocks(kLayerOut[l])), dim3(256), 0, st, m.vb[l].as<float>(),
 		                   static_cast<size_t>(kLayerOut[l]), 0.0f);
 		hipLaunchKernelGGL(k_to_bf16, dim3(blocks(n)), dim3(256), 0, st, m.w[l].as<float>(), n, m.wt_bf[l].as<uint16_t>(),
-		                   m.w_bf[l].as<uint16_t>(), kLayerOut[l], kLayerIn[l]);
+		                   m.w_bf[l].as<uint16_t>(), m.wt_frag[l].as<uint16_t>(), kLayerOut[l], kLayerIn[l]);
 	}
 	m.step = 0;
 	m.ready = true;
@@ -868,7 +1042,7 @@ hipError_t mlp_refresh_bf16(Mlp &m, hipStream_t st) {
 	for (int l = 0; l < 4; ++l) {
 		const size_t n = static_cast<size_t>(kLayerOut[l]) * kLayerIn[l];
 		hipLaunchKernelGGL(k_to_bf16, dim3(blocks(n)), dim3(256), 0, st, m.w[l].as<float>(), n, m.wt_bf[l].as<uint16_t>(),
-		                   m.w_bf[l].as<uint16_t>(), kLayerOut[l], kLayerIn[l]);
+		                   m.w_bf[l].as<uint16_t>(), m.wt_frag[l].as<uint16_t>(), kLayerOut[l], kLayerIn[l]);
 	}
 	return hipGetLastError();
 }
@@ -900,7 +1074,7 @@ static FusedArgs fused_args(const Mlp &m, const float *rays, uint64_t first, int
 		f.w[l] = m.wt_bf[l].as<uint16_t>();
 		f.b[l] = m.b[l].as<float>();
 	}
-	f.top4 = nullptr;
+	f.seeds = nullptr;
 	return f;
 }
 
@@ -927,8 +1101,17 @@ hipError_t mlp_forward_logits(Mlp &m, const float *rays, uint64_t first, int row
 hipError_t mlp_infer_top4(Mlp &m, const float *rays, uint64_t first, int rows, uint32_t *top4, hipStream_t st) {
 	if (rows <= 0) return hipSuccess;
 	FusedArgs f = fused_args(m, rays, first, rows);
-	f.top4 = top4;
+	f.seeds = top4;
 	hipLaunchKernelGGL(k_mlp_top4, dim3((rows + kFRows - 1) / kFRows), dim3(256), 0, st, f);
+	return hipGetLastError();
+}
+
+hipError_t mlp_infer_top1(Mlp &m, const float *rays, uint64_t first, int rows, uint32_t *top1, hipStream_t st) {
+	if (rows <= 0) return hipSuccess;
+	FusedArgs f = fused_args(m, rays, first, rows);
+	for (int l = 0; l < 4; ++l) f.w[l] = m.wt_frag[l].as<uint16_t>();
+	f.seeds = top1;
+	hipLaunchKernelGGL(k_mlp_top1, dim3(blocks(rows, kTop1Rows)), dim3(256), 0, st, f);
 	return hipGetLastError();
 }
 
@@ -993,10 +1176,10 @@ hipError_t mlp_backward(Mlp &m, const uint32_t *labels, int rows, float lr, hipS
 			PRT_TRY((gemm<E_MASK_BF16, 64, 64>(d, 1, st)));
 		}
 		a.w[l] = {m.w[l].as<float>(), m.gw[l].as<float>(), m.mw[l].as<float>(), m.vw[l].as<float>(), split, kSplits,
-		          m.wt_bf[l].as<uint16_t>(), m.w_bf[l].as<uint16_t>(), out, in, n_blocks};
+		          m.wt_bf[l].as<uint16_t>(), m.w_bf[l].as<uint16_t>(), m.wt_frag[l].as<uint16_t>(), out, in, n_blocks};
 		n_blocks += static_cast<unsigned>(in / 64) * (out / 32);
 		a.b[l] = {m.b[l].as<float>(), m.gb[l].as<float>(), m.mb[l].as<float>(), m.vb[l].as<float>(), colsum, static_cast<int>(row_tiles),
-		          nullptr, nullptr, out, l == 3 ? kMlpOut : out, n_blocks};  // the padding logits' bias stays
+		          nullptr, nullptr, nullptr, out, l == 3 ? kMlpOut : out, n_blocks};  // the padding logits' bias stays
 		n_blocks += blocks(out);
 		split += kSplits * kLayerWeights[l];
 		colsum += static_cast<size_t>(row_tiles) * out;

@@ -626,7 +626,9 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<S
 					// distance; the root traversal afterwards covers every triangle except those
 					// of the clusters already searched. The best cluster's box is not tested:
 					// the leaf test is exact, so a ray that misses it only visits its entry.
-					const uint4 s4 = reinterpret_cast<const uint4 *>(a.seeds)[ray_idx];  // best first
+					uint4 s4 = make_uint4(0u, 0u, 0u, 0u);  // best first
+					if (MULTI) s4 = reinterpret_cast<const uint4 *>(a.seeds)[ray_idx];
+					else s4.x = a.seeds[ray_idx];
 					sd[0] = s4.x < a.n_clusters ? a.cl_entry[s4.x] : 0u;
 					if (sd[0] == 0u) sd[0] = kInvalid;  // no seed, or the cluster is the whole tree
 					uint32_t key[4] = {};

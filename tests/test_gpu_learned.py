@@ -66,6 +66,20 @@ def test_top4_matches_full_logits(gpu_ctx, room):
     check_top4(gpu_ctx, scenes.rays(4, stream=2, first=777, count=517))
 
 
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 129, 4097])
+def test_top1_matches_full_logits(gpu_ctx, room, n):
+    """The one-seed inference's cluster is the argmax of the full logits where the two best are
+    clearly apart: one ray, and full and ragged workgroups."""
+    rays = scenes.rays(4, stream=2, first=4321, count=n)
+    best = prt.mlp_top1(gpu_ctx, rays)
+    four, logits = prt.mlp_top4(gpu_ctx, rays, with_logits=True)
+    gap = np.partition(logits, -2, axis=1)[:, -2:]
+    clear = (gap[:, 1] - gap[:, 0]) > 1e-3 * np.abs(gap[:, 1]).clip(1e-3)
+    assert clear.mean() > 0.9
+    assert np.array_equal(best[clear], logits.argmax(axis=1)[clear].astype(np.uint32))
+    assert np.array_equal(best, four[:, 0])  # the same products in the same order
+
+
 def test_learned_traversal_identical_to_plain(gpu_ctx, room):
     import torch
     train = scenes.rays(4, stream=1, count=262144)
