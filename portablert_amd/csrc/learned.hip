@@ -430,7 +430,7 @@ int prt_mi355x_mlp_top4(prt_ctx *c, const float *rays, uint64_t n, uint32_t *top
 
 // The same for the best cluster alone, by the inference of the one-seed traversal.
 int prt_mi355x_mlp_top1(prt_ctx *c, const float *rays, uint64_t n, uint32_t *top1) {
-	if (!c || !rays || !top1 || n == 0 || n > 65536) return PRT_ERR_ARG;
+	if (!c || !rays || !top1 || n == 0 || n > (1u << 20)) return PRT_ERR_ARG;
 	if (int r = check_learned(c)) return r;
 	DevBuf dr, dt;
 	hipError_t e = dr.ensure(n * 24);

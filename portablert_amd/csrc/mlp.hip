@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -44,9 +45,14 @@ __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float(stati
 
 // Place of weight (row, col) of a W^T [rows][cols] in its fragment order: 16 rows x 32 columns follow
 // each other as the MFMA operand of 64 lanes x 8 values, so a wave loads a fragment as 1 KB in a row.
+// Of 32 rows, tile 0 holds rows 0-3, 8-11, 16-19, 24-27 and tile 1 the others: a lane's results of the
+// two tiles are then 8 consecutive rows, which is its operand in the next layer.
 __device__ __forceinline__ size_t fragment_at(int row, int col, int cols) {
-	return (static_cast<size_t>(row >> 4) * (cols >> 5) + (col >> 5)) * 512 + ((((col >> 3) & 3) << 4) | (row & 15)) * 8 + (col & 7);
+	const int tile = (row >> 5) * 2 + ((row >> 2) & 1), at = ((row >> 3) & 3) * 4 + (row & 3);
+	return (static_cast<size_t>(tile) * (cols >> 5) + (col >> 5)) * 512 + ((((col >> 3) & 3) << 4) | at) * 8 + (col & 7);
 }
+// First of the 4 rows that a lane of group quad (lane / 16) holds of the results of a tile.
+__device__ __forceinline__ int fragment_row(int tile, int quad) { return (tile >> 1) * 32 + quad * 8 + (tile & 1) * 4; }
 
 enum Epi : int {
 	E_BIAS_F32 = 0,   // out f32 = acc + bias[n]
@@ -182,6 +188,10 @@ __global__ __launch_bounds__(kThreads) void k_gemm(GemmArgs g) {
 // 16 frequencies 2^(j/2) * pi, sin and cos: 192 features, bf16, in the order (input, frequency,
 // sin/cos).
 
+__device__ __forceinline__ uint32_t encode_pair(float y) {
+	return static_cast<uint32_t>(f2bf(__builtin_amdgcn_sinf(y))) | (static_cast<uint32_t>(f2bf(__builtin_amdgcn_cosf(y))) << 16);
+}
+
 // Inputs a0..a0+2, frequencies j0..j0+7 of one ray, each (sin, cos) pair as one 32-bit store: four
 // threads per ray.
 __device__ __forceinline__ void encode_quarter(const float *r, float4 lo, float4 inv_ext, int a0, int j0, uint16_t *o) {
@@ -202,8 +212,7 @@ __device__ __forceinline__ void encode_quarter(const float *r, float4 lo, float4
 		for (int jj = 0; jj < 8; ++jj) {
 			const int j = j0 + jj;  // v_sin/v_cos take revolutions: sin(2 pi y), y = in * 2^(j/2) / 2
 			const float y = in[q] * (0.5f * exp2f(0.5f * static_cast<float>(j)));
-			o32[(a0 + q) * 16 + j] = static_cast<uint32_t>(f2bf(__builtin_amdgcn_sinf(y))) |
-			                         (static_cast<uint32_t>(f2bf(__builtin_amdgcn_cosf(y))) << 16);
+			o32[(a0 + q) * 16 + j] = encode_pair(y);
 		}
 	}
 }
@@ -605,7 +614,6 @@ __device__ __forceinline__ void load_rays(const uint16_t *X, int lane, bf16x8 (&
 template <int K>
 __device__ __forceinline__ void hidden_layer_t(uint16_t *X, const uint16_t *wt, const float *bias, int lane, int wave) {
 	constexpr int RT = kRayTiles, KS = K / kBK;
-	const int n0 = wave * 64;  // this wave's 64 neurons
 	const uint16_t *wsrc = wt + static_cast<size_t>(wave * 4 * KS) * 512 + lane * 8;
 	bf16x8 w[KS], xr[RT][KS];
 #pragma unroll
@@ -617,7 +625,7 @@ __device__ __forceinline__ void hidden_layer_t(uint16_t *X, const uint16_t *wt, 
 		f32x4 acc[RT];
 #pragma unroll
 		for (int i = 0; i < RT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-		const int n = n0 + t * 16 + (lane >> 4) * 4;
+		const int n = fragment_row(wave * 4 + t, lane >> 4);
 		const f32x4 b = *reinterpret_cast<const f32x4 *>(bias + n);
 #pragma unroll
 		for (int kk = 0; kk < KS; ++kk) {
@@ -649,7 +657,7 @@ __global__ __launch_bounds__(256, 2) void k_mlp_top1(FusedArgs a) {
 	hidden_layer_t<kMlpHidden>(X, a.w[1], a.b[1], lane, wave);
 	hidden_layer_t<kMlpHidden>(X, a.w[2], a.b[2], lane, wave);
 	const uint16_t *wsrc = a.w[3] + wave * KS * 512 + lane * 8;
-	const float *bsrc = a.b[3] + wave * 16 + quad * 4;
+	const float *bsrc = a.b[3] + fragment_row(wave, quad);
 	bf16x8 w[KS], xr[RT][KS];
 #pragma unroll
 	for (int kk = 0; kk < KS; ++kk) w[kk] = *reinterpret_cast<const bf16x8 *>(wsrc + kk * 512);
@@ -691,14 +699,14 @@ __global__ __launch_bounds__(256, 2) void k_mlp_top1(FusedArgs a) {
 		}
 	};
 	f32x4 acc0[RT], acc1[RT], b0, b1;
-	step(0, acc0, b0, acc1, b1, true);
+	step(0, acc0, b0, acc1, b0, true);
 	for (int t = 1; t < kTiles; t += 2) {
 		step(t, acc1, b1, acc0, b0, false);
 		step(t + 1, acc0, b0, acc1, b1, false);
 	}
 #pragma unroll
 	for (int e = 0; e < 4; ++e) {  // the last tile's padding neurons are never taken
-		if ((kTiles - 1) * kFCols + wave * 16 + quad * 4 + e < kMlpOut) {
+		if ((kTiles - 1) * kFCols + fragment_row(wave, quad) + e < kMlpOut) {
 #pragma unroll
 			for (int i = 0; i < RT; ++i) take(i, e, acc0[i][e] + b0[e], (kTiles - 1) * 4);
 		}
@@ -710,7 +718,7 @@ __global__ __launch_bounds__(256, 2) void k_mlp_top1(FusedArgs a) {
 #pragma unroll
 	for (int i = 0; i < RT; ++i) {
 		float x = best[i];
-		uint32_t n = code[i] == 0xFFFFFFFFu ? code[i] : (code[i] >> 2) * kFCols + wave * 16 + quad * 4 + (code[i] & 3u);
+		uint32_t n = code[i] == 0xFFFFFFFFu ? code[i] : (code[i] >> 2) * kFCols + fragment_row(wave, quad) + (code[i] & 3u);
 #pragma unroll
 		for (int m = 16; m < 64; m *= 2) {
 			const float ox = __shfl_xor(x, m);
@@ -739,6 +747,203 @@ __global__ __launch_bounds__(256, 2) void k_mlp_top1(FusedArgs a) {
 			}
 		}
 		a.seeds[r0 + tid] = n;
+	}
+}
+
+// Many rays: a wave takes 64 rays through the whole network by itself, and a workgroup's four waves
+// share the weights, which pass through two LDS buffers of two 16-neuron tiles each (a barrier per
+// pair of tiles), so 256 rays cost one stream of weights from L2 instead of four. Activations never
+// leave the wave's registers: a lane computes its own operand of the encoding, and its results of a
+// hidden layer's two tiles are its operand of the next layer (the order of the fragments). The
+// hidden layers take 32 rays at a time, whose inputs and outputs fit the registers together. 1 Mi
+// rays: 1.78 ms (1.45 PFLOP/s) against 1.93 in k_mlp_top1; two waves a SIMD, whose comparisons (four
+// vector instructions a logit, about as many cycles as the products) are not hidden entirely.
+constexpr int kManyRows = 256;
+constexpr int kBiasAt[4] = {0, kMlpHidden, 2 * kMlpHidden, 3 * kMlpHidden};
+constexpr int kPairs = (kMlpOut - 1) / 32;  // pairs of output tiles before the one that holds the miss logit
+static_assert(kMlpOut == kPairs * 32 + 1 && kPairs % 2 == 0 && kMlpOutPad >= kPairs * 32 + 32, "output tiles");
+
+__global__ __launch_bounds__(256, 2) void k_mlp_top1_many(FusedArgs a) {
+	constexpr int KS = kMlpHidden / kBK, KS0 = kMlpIn / kBK;
+	__shared__ __align__(16) uint16_t W[2][2 * KS * 512];
+	__shared__ __align__(16) float bias[kBiasAt[3] + kPairs * 32 + 32];
+	const uint32_t tid = threadIdx.x;
+	const int lane = tid & 63, wave = tid >> 6, quad = lane >> 4;
+	const int r0 = blockIdx.x * kManyRows + wave * 64 + (lane & 15);
+	u32x4 pre[KS / 2];
+	auto fetch = [&](const uint16_t *src, int ks) {  // the weights of two tiles, ks fragments each
+		uint32_t zero = 0u;  // hidden from the compiler, which else keeps all layers' addresses across the loop below
+		asm volatile("" : "+s"(zero));
+		src += zero;
+#pragma unroll
+		for (int c = 0; c < KS / 2; ++c)
+			if (c < ks / 2) pre[c] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint8_t *>(src + c * 2048) + tid * 16u);
+	};
+	auto store = [&](uint16_t *dst, int ks) {
+#pragma unroll
+		for (int c = 0; c < KS / 2; ++c)
+			if (c < ks / 2) *reinterpret_cast<u32x4 *>(dst + (c * 256 + tid) * 8) = pre[c];
+	};
+	auto frag = [&](const uint16_t *w, int f) { return *reinterpret_cast<const bf16x8 *>(w + f * 512 + lane * 8); };
+	fetch(a.w[0], KS0);
+#pragma unroll
+	for (int l = 0; l < 3; ++l) bias[kBiasAt[l] + tid] = a.b[l][tid];
+	for (uint32_t k = tid; k < kPairs * 32 + 32; k += 256) bias[kBiasAt[3] + k] = a.b[3][k];
+	store(W[0], KS0);
+	__syncthreads();
+
+	bf16x8 lo[2][KS], hi[2][KS];  // the last hidden layer of rays 0-31 and 32-63
+	// one hidden layer; W[0] holds its first pair of tiles, and the next layer's at the end
+	auto layer = [&](auto ks_, const auto &in, bf16x8 (&out)[2][KS], const uint16_t *w, const float *b, const uint16_t *next, int next_ks) {
+		constexpr int ks = decltype(ks_)::value;
+#pragma unroll
+		for (int p = 0; p < KS; ++p) {
+			if (p + 1 < KS) fetch(w + (p + 1) * 2 * ks * 512, ks);
+			else fetch(next, next_ks);
+			f32x4 acc[2][2];  // tile, ray tile
+#pragma unroll
+			for (int t = 0; t < 2; ++t)
+#pragma unroll
+				for (int i = 0; i < 2; ++i) acc[t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+			for (int kk = 0; kk < ks; ++kk)
+#pragma unroll
+				for (int t = 0; t < 2; ++t) {
+					const bf16x8 f = frag(W[p & 1], t * ks + kk);
+#pragma unroll
+					for (int i = 0; i < 2; ++i) acc[t][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f, in[i][kk], acc[t][i], 0, 0, 0);
+				}
+			store(W[(p + 1) & 1], p + 1 < KS ? ks : next_ks);
+			union {
+				uint32_t u[4];
+				bf16x8 v;
+			} o[2];
+#pragma unroll
+			for (int t = 0; t < 2; ++t) {
+				const f32x4 bt = *reinterpret_cast<const f32x4 *>(b + fragment_row(2 * p + t, quad));
+#pragma unroll
+				for (int i = 0; i < 2; ++i)
+#pragma unroll
+					for (int h = 0; h < 2; ++h)
+						o[i].u[t * 2 + h] = f2bf(fmaxf(acc[t][i][2 * h] + bt[2 * h], 0.0f)) |
+						                    static_cast<uint32_t>(f2bf(fmaxf(acc[t][i][2 * h + 1] + bt[2 * h + 1], 0.0f))) << 16;
+			}
+#pragma unroll
+			for (int i = 0; i < 2; ++i) out[i][p] = o[i].v;
+			__syncthreads();
+		}
+	};
+#pragma unroll 1
+	for (int half = 0; half < 2; ++half) {
+#pragma unroll
+		for (int i = 0; i < 2; ++i)
+#pragma unroll
+			for (int kk = 0; kk < KS; ++kk) lo[i][kk] = hi[i][kk];
+		bf16x8 x[2][KS0], h[2][KS];
+#pragma unroll
+		for (int i = 0; i < 2; ++i) {
+			const int row = min(r0 + (half * 2 + i) * 16, a.rows - 1);
+			const float *r = a.rays + 6 * (a.first + row);
+			float in[6];
+			in[0] = (r[0] - a.lo.x) * a.inv_ext.x * 2.0f - 1.0f;
+			in[1] = (r[1] - a.lo.y) * a.inv_ext.y * 2.0f - 1.0f;
+			in[2] = (r[2] - a.lo.z) * a.inv_ext.z * 2.0f - 1.0f;
+			in[3] = r[3];
+			in[4] = r[4];
+			in[5] = r[5];
+#pragma unroll
+			for (int kk = 0; kk < KS0; ++kk) {
+				union {
+					uint32_t u[4];
+					bf16x8 v;
+				} o;
+#pragma unroll
+				for (int q = 0; q < 4; ++q) {
+					const float y = in[kk] * (0.5f * exp2f(0.5f * static_cast<float>(quad * 4 + q)));
+					o.u[q] = encode_pair(y);
+				}
+				x[i][kk] = o.v;
+			}
+		}
+		constexpr auto k0 = std::integral_constant<int, KS0>();
+		constexpr auto k1 = std::integral_constant<int, KS>();
+		layer(k0, x, hi, a.w[0], bias + kBiasAt[0], a.w[1], KS);
+		layer(k1, hi, h, a.w[1], bias + kBiasAt[1], a.w[2], KS);
+		layer(k1, h, hi, a.w[2], bias + kBiasAt[2], half == 0 ? a.w[0] : a.w[3], KS);
+	}
+
+	float best[4];
+	uint32_t code[4];  // tile * 4 + element
+#pragma unroll
+	for (int i = 0; i < 4; ++i) {
+		best[i] = -__builtin_inff();
+		code[i] = 0xFFFFFFFFu;
+	}
+	auto take = [&](int i, int e, float x, uint32_t c) {  // strict: the lower neuron at equal logits
+		const bool more = x > best[i];
+		best[i] = more ? x : best[i];
+		code[i] = more ? c + e : code[i];
+	};
+	bf16x8 f[4];
+	// tile t's MFMAs from fragments w, w + 1, .. with the comparisons of tile t - 1's results between them
+	auto tile = [&](const uint16_t *w, int first, int last, f32x4 (&acc)[4], const f32x4 (&old)[4], const f32x4 &ob, uint32_t c, bool compare) {
+#pragma unroll
+		for (int kk = 0; kk < KS; ++kk) {
+			const int p = first + kk;
+#pragma unroll
+			for (int i = 0; i < 4; ++i)
+				acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[p & 3], i < 2 ? lo[i & 1][kk] : hi[i & 1][kk],
+				                                                 kk == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[i], 0, 0, 0);
+			if (p + 4 < last) f[p & 3] = frag(w, p + 4);
+			if (compare) {
+#pragma unroll
+				for (int q = 0; q < 2; ++q) {
+					const int at = kk * 2 + q;
+					take(at / 4, at % 4, old[at / 4][at % 4] + ob[at % 4], c);
+				}
+			}
+			__builtin_amdgcn_sched_barrier(0);
+		}
+	};
+	f32x4 acc0[4], acc1[4], b0, b1;
+#pragma unroll
+	for (int i = 0; i < 4; ++i) acc1[i] = f32x4{-__builtin_inff(), -__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
+	b1 = f32x4{0.f, 0.f, 0.f, 0.f};
+	const float *bo = bias + kBiasAt[3] + quad * 8;
+	for (int p = 0; p < kPairs; ++p) {
+		const uint16_t *w = W[p & 1];
+		fetch(a.w[3] + static_cast<size_t>(p + 1) * 2 * KS * 512, KS);
+#pragma unroll
+		for (int q = 0; q < 4; ++q) f[q] = frag(w, q);
+		b0 = *reinterpret_cast<const f32x4 *>(bo + p * 32);
+		__builtin_amdgcn_sched_barrier(0);
+		tile(w, 0, 2 * KS, acc0, acc1, b1, static_cast<uint32_t>(2 * p - 1) * 4u, true);
+		b1 = *reinterpret_cast<const f32x4 *>(bo + p * 32 + 4);
+		tile(w, KS, 2 * KS, acc1, acc0, b0, static_cast<uint32_t>(2 * p) * 4u, true);
+		store(W[(p + 1) & 1], KS);
+		__syncthreads();
+	}
+#pragma unroll
+	for (int q = 0; q < 4; ++q) f[q] = frag(W[0], q);
+	tile(W[0], 0, KS, acc0, acc1, b1, static_cast<uint32_t>(2 * kPairs - 1) * 4u, true);
+	if (quad == 0) {  // the miss logit; the rest of the tile is padding
+#pragma unroll
+		for (int i = 0; i < 4; ++i) take(i, 0, acc0[i][0] + bo[kPairs * 32], static_cast<uint32_t>(2 * kPairs) * 4u);
+	}
+#pragma unroll
+	for (int i = 0; i < 4; ++i) {  // the best of a ray's four lanes
+		float x = best[i];
+		uint32_t n = code[i] == 0xFFFFFFFFu ? code[i] : fragment_row(static_cast<int>(code[i] >> 2), quad) + (code[i] & 3u);
+#pragma unroll
+		for (int m = 16; m < 64; m *= 2) {
+			const float ox = __shfl_xor(x, m);
+			const uint32_t on = __shfl_xor(n, m);
+			if (top_better(ox, on, x, n)) {
+				x = ox;
+				n = on;
+			}
+		}
+		if (quad == 0 && r0 + i * 16 < a.rows) a.seeds[r0 + i * 16] = n;
 	}
 }
 
@@ -993,6 +1198,10 @@ hipError_t gemm(const GemmArgs &g, int splits, hipStream_t st) {
 
 // ------------------------------------------------------------------------------ host side
 
+// Rows below which k_mlp_top1 runs: its workgroups of 64 rays fill the chip earlier. It against
+// k_mlp_top1_many, in us: 65,536 rays 125 / 149, 262,144 rays 485 / 455, 1 Mi rays 1,930 / 1,780.
+constexpr int kManyFrom = 262144;
+
 const int kLayerIn[4] = {kMlpIn, kMlpHidden, kMlpHidden, kMlpHidden};
 const int kLayerOut[4] = {kMlpHidden, kMlpHidden, kMlpHidden, kMlpOutPad};
 
@@ -1111,7 +1320,8 @@ hipError_t mlp_infer_top1(Mlp &m, const float *rays, uint64_t first, int rows, u
 	FusedArgs f = fused_args(m, rays, first, rows);
 	for (int l = 0; l < 4; ++l) f.w[l] = m.wt_frag[l].as<uint16_t>();
 	f.seeds = top1;
-	hipLaunchKernelGGL(k_mlp_top1, dim3(blocks(rows, kTop1Rows)), dim3(256), 0, st, f);
+	if (rows < kManyFrom) hipLaunchKernelGGL(k_mlp_top1, dim3(blocks(rows, kTop1Rows)), dim3(256), 0, st, f);
+	else hipLaunchKernelGGL(k_mlp_top1_many, dim3(blocks(rows, kManyRows)), dim3(256), 0, st, f);
 	return hipGetLastError();
 }
 

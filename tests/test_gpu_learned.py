@@ -69,7 +69,7 @@ def test_top4_matches_full_logits(gpu_ctx, room):
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 129, 4097])
 def test_top1_matches_full_logits(gpu_ctx, room, n):
     """The one-seed inference's cluster is the argmax of the full logits where the two best are
-    clearly apart: one ray, and full and ragged workgroups."""
+    clearly apart: one ray, full and ragged workgroups."""
     rays = scenes.rays(4, stream=2, first=4321, count=n)
     best = prt.mlp_top1(gpu_ctx, rays)
     four, logits = prt.mlp_top4(gpu_ctx, rays, with_logits=True)
@@ -78,6 +78,16 @@ def test_top1_matches_full_logits(gpu_ctx, room, n):
     assert clear.mean() > 0.9
     assert np.array_equal(best[clear], logits.argmax(axis=1)[clear].astype(np.uint32))
     assert np.array_equal(best, four[:, 0])  # the same products in the same order
+
+
+@pytest.mark.parametrize("n", [262143, 262144, 262145, 262400])
+def test_top1_many_rays(gpu_ctx, room, n):
+    """The kernels of few and of many rays around the line between them: the last rays, whose
+    workgroups are ragged or full, have the best of their top 4."""
+    rays = scenes.rays(4, stream=2, first=4321, count=n)
+    best = prt.mlp_top1(gpu_ctx, rays)
+    at = np.r_[0:1024, n - 1024:n]
+    assert np.array_equal(best[at], prt.mlp_top4(gpu_ctx, rays[at])[:, 0])
 
 
 def test_learned_traversal_identical_to_plain(gpu_ctx, room):
