@@ -177,7 +177,7 @@ class Context:
     def nearest_hits(self, rays, mask=mask_of(ALL_TAGS)):
         rays = np.ascontiguousarray(rays, np.float32).reshape(-1, 6)
         size, off = layout(mask)
-        out = np.zeros(len(rays), hit_dtype(mask))
+        out = np.empty(len(rays), hit_dtype(mask))  # every byte of every record is written
         offs = np.asarray(off, np.int32)
         self._check(lib().prt_mi355x_nearest_hits(self.h, _p(rays), len(rays), mask, _p(out), size, _p(offs)))
         return out

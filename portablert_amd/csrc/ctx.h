@@ -29,14 +29,15 @@ struct prt_ctx {
 	prt::TraceParams tp;
 	prt::TraceScratch ts;
 	prt::DevBuf rays_stage, out_stage;
-	// host-buffer entry point, in chunks: pinned double buffers, copy threads, and the streams
-	// that move data while the context's stream traces (created at the first large call)
+	// host-buffer entry point: pinned buffers, and for large calls in chunks copy threads and the
+	// streams that move data while the context's stream traces (created when first needed)
 	std::unique_ptr<prt::CopyPool> pool;
 	void *pin_in[2] = {nullptr, nullptr}, *pin_out[2] = {nullptr, nullptr};
-	size_t pin_in_bytes = 0, pin_out_bytes = 0;
+	size_t pin_in_bytes[2] = {0, 0}, pin_out_bytes[2] = {0, 0};
 	hipStream_t s_in = nullptr, s_out = nullptr;
 	hipEvent_t ev_in[2] = {nullptr, nullptr}, ev_tr[2] = {nullptr, nullptr}, ev_out[2] = {nullptr, nullptr};
 	prt::DevBuf chunk_err;
+	bool host_called = false;  // a host-buffer call of one launch has been made
 	bool has_scene = false;
 	// traversal without allocation: result of the scratch address look-up at creation, and
 	// whether this context has launched with that scratch (its error flags live there)

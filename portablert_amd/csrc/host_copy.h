@@ -18,6 +18,7 @@ namespace prt {
 
 class CopyPool {
   public:
+	static constexpr size_t kSplitBytes = size_t{4} << 20;  // smaller copies are one memcpy
 	explicit CopyPool(int threads) : n_(std::max(1, threads)) {
 		try {
 			for (int i = 1; i < n_; ++i) th_.emplace_back([this, i] { loop(i); });
@@ -39,7 +40,7 @@ class CopyPool {
 
 	// Copies `bytes` from src to dst, split across the pool; returns when all parts are done.
 	void copy(void *dst, const void *src, size_t bytes) {
-		if (n_ == 1 || bytes < (size_t{4} << 20)) {
+		if (n_ == 1 || bytes < kSplitBytes) {
 			std::memcpy(dst, src, bytes);
 			return;
 		}
