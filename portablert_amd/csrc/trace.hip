@@ -48,6 +48,7 @@ struct KArgs {
 	uint32_t chunk;         // rays a wave reserves per atomic
 	uint32_t leaf_phase;    // triangle phase once parked lanes >= live lanes * leaf_phase / 64
 	uint32_t wide_grid;     // workgroups of k_trace_wide for the first pass, 0: k_trace
+	uint32_t wide_rest;     // of the second pass, 0: k_trace
 	uint32_t refill;        // load new rays once at least this many lanes are idle (or all are)
 	float margin_rel;
 	float margin_abs;
@@ -800,7 +801,8 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<S
 // the sorting network), all pushes are one LDS store, and near and far planes are picked by
 // address. A wave holds 8 rays, each traversed at its own pace: pop, node test and leaf test in
 // one iteration. Costs more issue slots per ray than k_trace, which takes larger launches. 65,536
-// rays: room 137 -> 102 us, 1.5 M-triangle soup 510 -> 325, icosphere camera 153 -> 90.
+// rays: room 137 -> 102 us, 1.5 M-triangle soup 510 -> 325, icosphere camera 153 -> 90. kRest, the second
+// pass, tests its lane's child by the reference formula.
 constexpr int kWideStack = 32;   // LDS stack entries per ray; deeper ones in the spill array
 constexpr int kWidePad = 33;     // entry stride of a ray's stack (the groups' tops in different banks)
 constexpr int kWideBlock = 128;
@@ -830,12 +832,16 @@ __device__ __forceinline__ void wide_best(WideHit &h) {
 	if (better(t, id, h.t, h.id)) h = {t, u, v, id};
 }
 
-template <int MODE, bool NC>
-__global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_trace_wide(KArgs a) {
+template <int MODE, bool NC, int PASS>
+__global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(PASS == kFast ? 8 : 6))) void k_trace_wide(KArgs a) {
 	static_assert(MODE == kPlain || MODE == kWatertight, "one scene, no seeds");
 	__shared__ uint2 lds[kWideBlock / 8][kWidePad];
-	if (blockIdx.x == 0 && threadIdx.x < kCounters && a.next) a.next[threadIdx.x] = 0ull;
 	uint32_t *flags = reinterpret_cast<uint32_t *>(a.counter + C_ERR);  // [0] errors, [1] rays left to kRest
+	const uint32_t n_left = PASS == kRest ? flags[1] : 0u;
+	if (PASS == kRest && n_left == 0u) return;
+	if (PASS == kFast && blockIdx.x == 0 && threadIdx.x < kCounters && a.next) a.next[threadIdx.x] = 0ull;
+	const bool listed = PASS == kRest && n_left <= kLeftMax;
+	const uint64_t n_work = listed ? n_left : a.n_rays;
 	const uint8_t *nodes = static_cast<const uint8_t *>(a.nodes);
 	const uint32_t g = threadIdx.x & 7u, group = (blockIdx.x * kWideBlock + threadIdx.x) >> 3;
 	const uint32_t groups = gridDim.x * (kWideBlock / 8);
@@ -844,14 +850,14 @@ __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(8)))
 	bool told = false;  // the list of left rays is full
 	Ray r;
 	uint32_t near_at[3] = {0, 0, 0};  // byte of this lane's near bound on each axis, in the node
-	uint64_t ray_idx = group;
+	uint64_t work = group;
 	bool active = false;
 	uint32_t cur = kInvalid, sp = 0;
 	for (;;) {
-		const bool full = __ballot(told) != 0ull;  // the same in every lane
+		const bool full = PASS != kFast || __ballot(told) != 0ull;  // the same in every lane
 		// ---- a group without a ray takes its next one
-		if (!active && ray_idx < a.n_rays) {
-			load_ray<kFast, MODE == kWatertight>(a, ray_idx, a.margin_abs, a.fast_scene != 0, r);
+		if (!active && work < n_work) {
+			load_ray<PASS, MODE == kWatertight>(a, listed ? a.left[work] : work, a.margin_abs, a.fast_scene != 0, r);
 			active = r.mine;
 			const uint64_t left = __ballot(!active && g == 0u);
 			if (left != 0ull && !full) {  // to the second pass: one atomic for the wave's groups
@@ -865,15 +871,15 @@ __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(8)))
 				at = __builtin_amdgcn_readlane(at, lead);
 				told = at + n > kLeftMax;
 				const uint32_t k = at + static_cast<uint32_t>(__popcll(left & ((1ull << lane) - 1ull)));
-				if (!active && g == 0u && k < kLeftMax) a.left[k] = ray_idx;
+				if (!active && g == 0u && k < kLeftMax) a.left[k] = work;
 			}
-			if (!active) ray_idx += groups;
+			if (!active) work += groups;
 			cur = r.never || a.n_nodes == 0 ? kInvalid : 0u;
 			sp = 0;
 #pragma unroll
-			for (int ax = 0; ax < 3; ++ax) near_at[ax] = 32u + 8u * ax + (r.inv[ax] >= 0.0f ? 0u : 24u) + g;
+			for (int ax = 0; ax < 3; ++ax) near_at[ax] = 32u + 8u * ax + (PASS == kRest || r.inv[ax] >= 0.0f ? 0u : 24u) + g;
 		}
-		if (__ballot(active || ray_idx < a.n_rays) == 0ull) break;
+		if (__ballot(active || work < n_work) == 0ull) break;
 		if (!active) continue;
 		const float limit = cull_limit(r, a);
 		// ---- next entry: the nearest child of the last node, else the stack's top (culled again)
@@ -886,9 +892,9 @@ __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(8)))
 			}
 		}
 		if (cur == kInvalid) {  // ray finished
-			if (g == 0u) write_record(a, ray_idx, r);
+			if (g == 0u) write_record(a, listed ? a.left[work] : work, r);
 			active = false;
-			ray_idx += groups;
+			work += groups;
 			continue;
 		}
 		if (!(cur & kLeafBit)) {
@@ -899,31 +905,46 @@ __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(8)))
 			}
 			const uint8_t *node = nodes + static_cast<uint64_t>(cur) * sizeof(NodeQ);
 			const uint4 w0 = reinterpret_cast<const uint4 *>(node)[0], w1 = reinterpret_cast<const uint4 *>(node)[1];
-			uint32_t qn[3], qf[3];
+			uint32_t qn[3], qf[3];  // near and far bounds (kRest: low and high)
 #pragma unroll
 			for (int ax = 0; ax < 3; ++ax) {
 				qn[ax] = node[near_at[ax]];
-				qf[ax] = node[r.inv[ax] >= 0.0f ? near_at[ax] + 24u : near_at[ax] - 24u];
+				qf[ax] = node[PASS == kRest || r.inv[ax] >= 0.0f ? near_at[ax] + 24u : near_at[ax] - 24u];
 			}
 			const float p[3] = {__uint_as_float(w0.x), __uint_as_float(w0.y), __uint_as_float(w0.z)};
 			const uint32_t ncull = NC ? w0.w >> 24 : 0u;
-			float tn[3], tf[3];
-			// the one-fma bounds of ChildTest<NodeQ>, for this lane's child
-#pragma unroll
-			for (int ax = 0; ax < 3; ++ax) {
-				const float sc = exp2i(static_cast<int8_t>((w0.w >> (8 * ax)) & 0xFF));
-				const float step = sc * r.inv[ax];
-				const float base = (p[ax] - r.o[ax]) * r.inv[ax];
-				const float margin = (0x1p-18f * fabsf(r.inv[ax])) * fmaf(255.0f, sc, fabsf(p[ax]) + fabsf(r.o[ax]));
-				tn[ax] = fmaf(static_cast<float>(qn[ax]), step, base - margin);
-				tf[ax] = fmaf(static_cast<float>(qf[ax]), step, base + margin);
-			}
-			const float tmin = fmaxf(fmaxf(tn[0], tn[1]), tn[2]);
-			const float tmax = fminf(fminf(tf[0], tf[1]), tf[2]);
 			const float lim = ncull != 0u ? __builtin_inff() : limit;
 			const uint32_t meta = ((g < 4u ? w1.z : w1.w) >> (8u * (g & 3u))) & 0xFFu;
-			const bool hit = meta != kMetaEmpty && tmax >= 0.0f && tmin <= tmax && tmin <= lim;
-			uint32_t key = sort_key_finite(tmin, static_cast<int>(g));
+			float sc[3], tmin;
+#pragma unroll
+			for (int ax = 0; ax < 3; ++ax) sc[ax] = exp2i(static_cast<int8_t>((w0.w >> (8 * ax)) & 0xFF));
+			bool hit = meta != kMetaEmpty;
+			uint32_t key;
+			if constexpr (PASS == kFast) {  // the one-fma bounds of ChildTest<NodeQ>, for this lane's child
+				float tn[3], tf[3];
+#pragma unroll
+				for (int ax = 0; ax < 3; ++ax) {
+					const float step = sc[ax] * r.inv[ax];
+					const float base = (p[ax] - r.o[ax]) * r.inv[ax];
+					const float margin = (0x1p-18f * fabsf(r.inv[ax])) * fmaf(255.0f, sc[ax], fabsf(p[ax]) + fabsf(r.o[ax]));
+					tn[ax] = fmaf(static_cast<float>(qn[ax]), step, base - margin);
+					tf[ax] = fmaf(static_cast<float>(qf[ax]), step, base + margin);
+				}
+				tmin = fmaxf(fmaxf(tn[0], tn[1]), tn[2]);
+				const float tmax = fminf(fminf(tf[0], tf[1]), tf[2]);
+				hit = hit && tmax >= 0.0f && tmin <= tmax && tmin <= lim;
+				key = sort_key_finite(tmin, static_cast<int>(g));
+			} else {  // its reference formula
+				float lo[3], hi[3];
+#pragma unroll
+				for (int ax = 0; ax < 3; ++ax) {
+					lo[ax] = fmaf(static_cast<float>(qn[ax]), sc[ax], p[ax]);
+					hi[ax] = fmaf(static_cast<float>(qf[ax]), sc[ax], p[ax]);
+				}
+				tmin = child_slab<MODE == kWatertight>(slab_ray(r), lo, hi, lim, (ncull >> g) & 1u);
+				hit = hit && !__builtin_isnan(tmin);
+				key = sort_key(tmin, static_cast<int>(g));
+			}
 			if (NC && ((ncull >> g) & 1u)) key = kKeyNoCull | g;
 			if (!hit) key = kMiss;
 			// rank among the group's hits (keys differ in their slot bits)
@@ -1005,13 +1026,19 @@ void launch_nc(const KArgs &a, uint32_t grid, bool count, hipStream_t st) {
 		launch_pass<Node, S, B, MODE, NC, kAll>(a, grid, count, st);
 	} else {
 		if constexpr (MODE == kPlain || MODE == kWatertight) {
-			if (a.wide_grid) hipLaunchKernelGGL((k_trace_wide<MODE, NC>), dim3(a.wide_grid), dim3(kWideBlock), 0, st, a);
+			if (a.wide_grid) hipLaunchKernelGGL((k_trace_wide<MODE, NC, kFast>), dim3(a.wide_grid), dim3(kWideBlock), 0, st, a);
 			else launch_pass<Node, S, B, MODE, NC, kFast>(a, grid, count, st);
 		} else {
 			launch_pass<Node, S, B, MODE, NC, kFast>(a, grid, count, st);
 		}
 		// seeds do not change a record: the second pass of the learned modes is the plain one
 		constexpr int REST = MODE == kSeeded || MODE == kSeededMulti ? kPlain : MODE;
+		if constexpr (MODE == kPlain || MODE == kWatertight) {
+			if (a.wide_rest) {
+				hipLaunchKernelGGL((k_trace_wide<MODE, NC, kRest>), dim3(a.wide_rest), dim3(kWideBlock), 0, st, a);
+				return;
+			}
+		}
 		launch_pass<Node, S, B, REST, NC, kRest>(a, grid, count, st);
 	}
 }
@@ -1076,6 +1103,7 @@ struct TracePlan {
 	uint32_t spill_depth = 0;  // stack entries per thread kept in global memory
 	uint32_t chunk = 64;       // rays a wave reserves at a time
 	uint32_t wide_grid = 0;    // workgroups of k_trace_wide, 0: k_trace
+	uint32_t wide_rest = 0;    // of the second pass
 };
 
 // several: seeds or scenes, which only k_trace takes.
@@ -1111,9 +1139,14 @@ hipError_t plan_trace(const Bvh8 &b, TraceScratch &s, const TraceParams &p, uint
 	// rays 160 / 135, 519 / 369, 169 / 96; 131,072 rays 171 / 178, 535 / 555, 178 / 91. Watertight,
 	// 65,536 rays: 358 / 300, 1344 / 1211, 231 / 169; 131,072 rays 396 / 484, 1393 / 2021, 261 / 276.
 	const uint64_t resident = static_cast<uint64_t>(s.n_cus) * 32 * 8;
-	if (n <= (p.leaf_test == 1 ? resident : resident + resident / 2) && p.node_format != 0 && p.waves_per_cu <= 0 &&
-	    !p.count_stats && !several)
-		pl.wide_grid = static_cast<uint32_t>((std::min(n, resident) * 8 + kWideBlock - 1) / kWideBlock);
+	const bool wide = p.node_format != 0 && p.waves_per_cu <= 0 && !p.count_stats && !several;
+	const uint32_t wide_groups = static_cast<uint32_t>((std::min(n, resident) * 8 + kWideBlock - 1) / kWideBlock);
+	if (wide && n <= (p.leaf_test == 1 ? resident : resident + resident / 2)) pl.wide_grid = wide_groups;
+	// The second pass's reference formula is a longer chain for one lane: parallel rays along y (z for the
+	// icosphere), one lane against eight, in us: 4,096 rays 237 / 113, 448 / 171, 132 / 65; 65,536 rays 365 / 250, 619 /
+	// 350, 303 / 207; 131,072 rays 354 / 318, 687 / 499, 273 / 210; 262,144 rays 488 / 600, 796 / 920, 403 / 388.
+	// Watertight, the room: 4,096 rays 477 / 216, 131,072 rays 632 / 627, 262,144 rays 789 / 1,205.
+	if (wide && n <= 2 * resident) pl.wide_rest = wide_groups;
 	// stack bound: each visited node pushes at most 7 entries, so 7 * depth + 1 suffice
 	pl.max_entries = 7u * std::max(1u, b.depth) + 8u;
 	pl.spill_depth = pl.max_entries > static_cast<uint32_t>(S) ? pl.max_entries - S : 1u;
@@ -1124,7 +1157,7 @@ hipError_t plan_trace(const Bvh8 &b, TraceScratch &s, const TraceParams &p, uint
 uint64_t spill_entries(const TracePlan &pl, const TraceParams &p) {
 	const uint64_t one = static_cast<uint64_t>(pl.spill_depth) * pl.grid * p.block;
 	const uint64_t deep = pl.max_entries > static_cast<uint32_t>(kWideStack) ? pl.max_entries - kWideStack : 0u;
-	return std::max(one, deep * pl.wide_grid * (kWideBlock / 8));
+	return std::max(one, deep * std::max(pl.wide_grid, pl.wide_rest) * (kWideBlock / 8));
 }
 
 // Launches the traversal with the given counters (clear: not all 0 yet, cleared here by a kernel)
@@ -1156,6 +1189,7 @@ hipError_t run_trace(const Bvh8 &b, const TraceParams &p, const float *rays, uin
 	a.spill_depth = pl.spill_depth;
 	a.chunk = pl.chunk;
 	a.wide_grid = pl.wide_grid;
+	a.wide_rest = pl.wide_rest;
 	a.leaf_phase = static_cast<uint32_t>(std::max(1, std::min(64, p.leaf_phase)));
 	a.refill = static_cast<uint32_t>(std::max(1, std::min(64, p.refill)));
 	a.margin_rel = p.margin_rel;
@@ -1292,7 +1326,7 @@ hipError_t trace_bvh8_noalloc(const Bvh8 &b, TraceScratch &s, const TraceParams 
 	*need_bytes = kNoAllocCounterBytes + per_group;
 	if (fit == 0) return hipErrorInvalidValue;
 	pl.grid = static_cast<uint32_t>(std::min<uint64_t>(pl.grid, fit));
-	if (sizeof(uint2) * spill_entries(pl, p) > kNoAllocScratchBytes - kNoAllocCounterBytes) pl.wide_grid = 0;
+	if (sizeof(uint2) * spill_entries(pl, p) > kNoAllocScratchBytes - kNoAllocCounterBytes) pl.wide_grid = pl.wide_rest = 0;
 	uint8_t *base = static_cast<uint8_t *>(scratch_ptr);
 	return run_trace(b, p, rays, n, mask, out, st, reinterpret_cast<unsigned long long *>(base), true, nullptr,
 	                 reinterpret_cast<unsigned long long *>(base + kNoAllocScratchBytes),

@@ -61,3 +61,19 @@ def test_stack_deeper_than_lds(gpu_ctx):
         both(gpu_ctx, rays, oracle.brute(tris, rays), "deep")
     finally:
         gpu_ctx.set_option("cull", 1)
+
+
+@pytest.mark.parametrize("leaf_test", [0, 1])
+@pytest.mark.parametrize("n", [1, 4096, 4097, 65537, 98305, 131072, 131073])
+def test_second_pass(gpu_ctx, n, leaf_test):
+    """Rays with d_x = 0, which the second launch traces: listed, more than the list holds (4,096),
+    more than one round of groups, and where its eight lanes per ray end; an ordinary ray in every 7."""
+    tris, rays = soup(3000, 1), rays_in(n, n)
+    rays[np.arange(n) % 7 != 3, 3] = 0.0
+    gpu_ctx.set_tris(tris)
+    gpu_ctx.set_option("leaf_test", leaf_test)
+    try:
+        mode = oracle.LOWEST_ID | (oracle.WATERTIGHT if leaf_test else 0)
+        both(gpu_ctx, rays, oracle.trace(tris, rays, mode), f"n={n} leaf_test={leaf_test}")
+    finally:
+        gpu_ctx.set_option("leaf_test", 0)
