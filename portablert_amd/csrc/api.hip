@@ -403,8 +403,10 @@ static bool pageable(const void *p) {
 
 // One launch over rays and records in pageable memory. Up to kDirectRays rays the kernel itself reads
 // the rays from pinned memory and writes the records there. More pass through two pinned buffers in
-// up to four slices, the host copying one while the DMA engine moves the next.
-static int nearest_hits_staged(prt_ctx *c, const float *rays, uint64_t n, uint32_t mask, void *out, uint32_t stride) {
+// slices, the host copying one while the DMA engine moves the next. *no_memory: nothing was done, for want of
+// pinned memory.
+static int nearest_hits_staged(prt_ctx *c, const float *rays, uint64_t n, uint32_t mask, void *out, uint32_t stride,
+                               bool *no_memory) {
 	const uint64_t in_bytes = n * 24ull, out_bytes = n * static_cast<uint64_t>(stride);
 	const bool direct = n <= kDirectRays;
 	auto slice_of = [&](uint64_t bytes) {
@@ -415,6 +417,11 @@ static int nearest_hits_staged(prt_ctx *c, const float *rays, uint64_t n, uint32
 	for (int b = 0; b < (direct ? 1 : 2) && e == hipSuccess; ++b) {
 		e = ensure_pinned(c->pin_in[b], c->pin_in_bytes[b], in_slice);
 		if (e == hipSuccess) e = ensure_pinned(c->pin_out[b], c->pin_out_bytes[b], out_slice);
+	}
+	*no_memory = e != hipSuccess;
+	if (*no_memory) {
+		(void)hipGetLastError();
+		return PRT_OK;
 	}
 	for (int b = 0; b < 2 && e == hipSuccess && !direct; ++b) {
 		hipEvent_t *evs[2] = {&c->ev_in[b], &c->ev_out[b]};
@@ -495,10 +502,13 @@ int prt_mi355x_nearest_hits(prt_ctx *c, const float *rays, uint64_t n, uint32_t 
 		const bool again = c->host_called;
 		c->host_called = true;
 		if (again && pageable(rays) && pageable(out)) {
-			int r = nearest_hits_staged(c, rays, n, mask, out, stride);
-			if (r != PRT_OK) (void)hipStreamSynchronize(c->stream);  // nothing may still use the pinned buffers
-			else c->api_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-			return r;
+			bool no_memory = false;
+			const int r = nearest_hits_staged(c, rays, n, mask, out, stride, &no_memory);
+			if (!no_memory) {
+				if (r != PRT_OK) (void)hipStreamSynchronize(c->stream);  // nothing may still use the pinned buffers
+				else c->api_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+				return r;
+			}
 		}
 		e = hipMemcpyAsync(c->rays_stage.ptr, rays, n * 24ull, hipMemcpyHostToDevice, c->stream);
 		if (e != hipSuccess) return hip_fail(c, e, "nearest_hits: ray copy");
