@@ -756,8 +756,8 @@ __global__ __launch_bounds__(256, 2) void k_mlp_top1(FusedArgs a) {
 // leave the wave's registers: a lane computes its own operand of the encoding, and its results of a
 // hidden layer's two tiles are its operand of the next layer (the order of the fragments). The
 // hidden layers take 32 rays at a time, whose inputs and outputs fit the registers together. 1 Mi
-// rays: 1.78 ms (1.45 PFLOP/s) against 1.93 in k_mlp_top1; two waves a SIMD, whose comparisons (four
-// vector instructions a logit, about as many cycles as the products) are not hidden entirely.
+// rays: 1.78 ms (1.45 PFLOP/s) against 1.93 in k_mlp_top1. The comparisons hide behind the products:
+// with a quarter of them left out (the bias as the products' first addend) it took the same 1.78 ms.
 constexpr int kManyRows = 256;
 constexpr int kBiasAt[4] = {0, kMlpHidden, 2 * kMlpHidden, 3 * kMlpHidden};
 constexpr int kPairs = (kMlpOut - 1) / 32;  // pairs of output tiles before the one that holds the miss logit
