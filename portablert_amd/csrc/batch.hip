@@ -62,19 +62,18 @@ namespace {
 		if (e_ != hipSuccess) return e_;                                                           \
 	} while (0)
 
-// Per-scene culling margin (a fixed fraction of the scene extent, as for one scene) and the
-// one-fma node test flag (every vertex coordinate below 2^60 in magnitude).
+// Per-scene culling margin (a fixed fraction of the scene extent, as for one scene) and largest
+// vertex coordinate in magnitude.
 __global__ __launch_bounds__(256) void k_batch_info(const float *__restrict__ box, uint32_t scenes, int margin_log2,
                                                     float2 *__restrict__ info) {
 	const uint32_t s = blockIdx.x * 256 + threadIdx.x;
 	if (s >= scenes) return;
 	const float *b = box + 6ull * s;
-	float ext = 0.0f;
-	bool fast = true;
+	float ext = 0.0f, reach = 0.0f;
 	for (int k = 0; k < 3; ++k) ext = fmaxf(ext, b[3 + k] - b[k]);
-	for (int k = 0; k < 6; ++k) fast &= fabsf(b[k]) < 0x1p60f;
+	for (int k = 0; k < 6; ++k) reach = fmaxf(reach, fabsf(b[k]));
 	if (!__builtin_isfinite(ext)) ext = 0.0f;
-	info[s] = make_float2(ldexpf(ext, -margin_log2 - 6), fast ? 1.0f : 0.0f);
+	info[s] = make_float2(ldexpf(ext, -margin_log2 - 6), reach);
 }
 
 uint64_t scene_tris(const Batch &b, uint32_t s) { return b.tri_off[s + 1] - b.tri_off[s]; }

@@ -286,6 +286,43 @@ __host__ __device__ inline bool cull_unsafe(const float v[9]) {
 	return !(num <= 1000.0f * m * den);
 }
 
+// ---------------------------------------------------------------- rays of the one-fma node test
+//
+// The one-fma node test (ChildTest in trace.hip) moves the planes of a box apart by 2^-18 |1/d_k| len_k
+// on axis k, len_k = 255 * 2^e_k + |p_k| + |o_k| of the node, which has to cover the rounding of its own
+// products and of the reference formula's: 8 * 2^-24 of the same, while nothing overflows or
+// underflows.
+
+// Stands for 1/0 in that test on the y and z axes: a box that holds o_k must span every t there.
+constexpr float kFlat = 0x1p60f;
+
+// Whether every |1/d_k| is below 2^30 (or d_k is 0) and every |o_k| below 2^60 in a scene whose
+// largest coordinate, `reach`, is below 2^60: no product of the node test overflows. Distance culling
+// asks for the same (cull_unsafe).
+__host__ __device__ inline bool ray_in_range(const float o[3], const float d[3], const float inv[3], float reach) {
+	bool ok = reach < 0x1p60f;
+	for (int k = 0; k < 3; ++k) ok &= (d[k] == 0.0f || fabsf(inv[k]) < 0x1p30f) && fabsf(o[k]) < 0x1p60f;
+	return ok;
+}
+
+// Whether a ray in range may take the one-fma node test; others take the reference formula. Not with
+// d_x = 0 (child_slab in trace.hip). With d_y or d_z = 0 a box around o_k spans at least 7/8 of its
+// margin there, 2^42 len_k >= 2^42 |o_k|, and the t of the other axes reach (reach + |o|) max |1/d|, a
+// few parts in a hundred more for the grid's rounding: len_k knows nothing of those axes, so a box
+// thin on axis k near coordinate 0 would end before the hit. Such a ray is fast only if |o_k| alone
+// covers them (2^40, to spare).
+__host__ __device__ inline bool one_fma_ray(const float o[3], const float d[3], const float inv[3], float reach) {
+	float inv_max = 0.0f, o_max = 0.0f;
+	for (int k = 0; k < 3; ++k) {
+		if (d[k] != 0.0f) inv_max = fmaxf(inv_max, fabsf(inv[k]));
+		o_max = fmaxf(o_max, fabsf(o[k]));
+	}
+	const float t_max = (reach + o_max) * inv_max;
+	bool ok = d[0] != 0.0f;
+	for (int k = 1; k < 3; ++k) ok &= d[k] != 0.0f || 0x1p40f * fabsf(o[k]) >= t_max;
+	return ok;
+}
+
 // Keep the better of (t, id): smaller t, equal finite t resolved to the lower id. NaN and +inf
 // never win (the reference's strict t < t_near with t_near starting at +inf).
 __device__ __forceinline__ bool better(float t, uint32_t id, float tb, uint32_t idb) {

@@ -177,7 +177,7 @@ struct SeedArgs {
 
 // Several scenes in one launch over a BVH built from a SceneSet: rays are claimed in tiles
 // {first lo, first hi, count, scene} (each inside one scene), and info holds per scene
-// {absolute culling margin, 1 if every vertex is below 2^60 in magnitude else 0}. n is the total
+// {absolute culling margin, largest vertex coordinate in magnitude}. n is the total
 // ray count and records go to out + ray index * stride.
 struct BatchArgs {
 	const uint4 *tiles;

@@ -53,7 +53,7 @@ struct KArgs {
 	float margin_rel;
 	float margin_abs;
 	int cull;
-	int fast_scene;         // every vertex coordinate below 2^60 in magnitude
+	float reach;            // largest vertex coordinate of the scene in magnitude
 	// learned seeding (null when off): 4 cluster ids per ray, cluster entries and fp32 boxes
 	const uint32_t *seeds;
 	const uint32_t *cl_entry;
@@ -61,7 +61,7 @@ struct KArgs {
 	uint32_t n_clusters;
 	int n_seeds;            // predicted clusters searched first (1..4, the best ones)
 	// several scenes (null when off): ray tiles {first lo, first hi, count, scene} claimed one
-	// per atomic, and per scene {margin_abs, fast_scene}; BVH8 node s is the root of scene s
+	// per atomic, and per scene {margin_abs, reach}; BVH8 node s is the root of scene s
 	const uint4 *tiles;
 	uint32_t n_tiles;
 	const float2 *scene_info;
@@ -108,14 +108,8 @@ struct Ray {
 	bool never;        // no triangle can be hit: NaN in origin or direction, or no direction
 };
 
-// Stands for 1/0 in the one-fma node test. A box around o_k on a zero axis then spans at least
-// +-2^42 (|p| + |o| + extent) there (the test's own margin, 2^-18 |1/d|), which holds every t of
-// the other axes (|t| <= 2^30 times the same lengths); a box that o_k lies outside of by more than
-// 2^-18 of its coordinates is left before any of them. All products stay below 2^127.
-constexpr float kFlat = 0x1p60f;
-
 template <int PASS, bool WT>
-__device__ __forceinline__ void load_ray(const KArgs &a, uint64_t idx, float margin_abs, bool fast_scene, Ray &r) {
+__device__ __forceinline__ void load_ray(const KArgs &a, uint64_t idx, float margin_abs, float reach, Ray &r) {
 	const float *p = a.rays + 6 * idx;  // 4-byte aligned AoS records of 24 bytes
 #pragma unroll
 	for (int k = 0; k < 3; ++k) {
@@ -124,19 +118,15 @@ __device__ __forceinline__ void load_ray(const KArgs &a, uint64_t idx, float mar
 	}
 #pragma unroll
 	for (int k = 0; k < 3; ++k) r.inv[k] = 1.0f / r.d[k];  // IEEE division, as the reference
-	// every |d_k| 0 or above 2^-30 (|1/d| below 2^30), |o| below 2^60 in a scene within 2^60
-	const float big = 0x1p60f, inv_big = 0x1p30f;
 	const bool zero[3] = {r.d[0] == 0.0f, r.d[1] == 0.0f, r.d[2] == 0.0f};
-	bool nan = false, in_range = fast_scene;
+	bool nan = false;
 #pragma unroll
-	for (int k = 0; k < 3; ++k) {
-		nan |= __builtin_isnan(r.o[k]) || __builtin_isnan(r.d[k]);
-		in_range &= (zero[k] || fabsf(r.inv[k]) < inv_big) && fabsf(r.o[k]) < big;
-	}
+	for (int k = 0; k < 3; ++k) nan |= __builtin_isnan(r.o[k]) || __builtin_isnan(r.d[k]);
+	const bool in_range = ray_in_range(r.o, r.d, r.inv, reach);
 	// With NaN in the origin or the direction every t is NaN, which never wins; without a
 	// direction every determinant is 0 (Moller-Trumbore) or NaN (the watertight test).
 	r.never = nan || (zero[0] && zero[1] && zero[2]);
-	const bool fast = in_range && !zero[0];  // d_x = 0: the reference formula (child_slab)
+	const bool fast = in_range && one_fma_ray(r.o, r.d, r.inv, reach);
 	r.mine = PASS == kFast ? fast || r.never : !(fast || r.never);
 	// margin_abs / |d|, rounded up (1 + 2^-20 covers the reciprocal square root's error). An
 	// infinite margin turns distance culling off for this ray: culling is exact only for rays
@@ -609,10 +599,10 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<S
 				}
 				if (BATCH) {
 					const float2 si = a.scene_info[scene];
-					load_ray<PASS, MODE == kWatertight>(a, ray_idx, si.x, si.y != 0.0f, r);
+					load_ray<PASS, MODE == kWatertight>(a, ray_idx, si.x, si.y, r);
 					cur = scene;
 				} else {
-					load_ray<PASS, MODE == kWatertight>(a, ray_idx, a.margin_abs, a.fast_scene != 0, r);
+					load_ray<PASS, MODE == kWatertight>(a, ray_idx, a.margin_abs, a.reach, r);
 					cur = 0u;
 				}
 				if (r.never || a.n_nodes == 0) cur = kInvalid;
@@ -857,7 +847,7 @@ __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(PASS
 		const bool full = PASS != kFast || __ballot(told) != 0ull;  // the same in every lane
 		// ---- a group without a ray takes its next one
 		if (!active && work < n_work) {
-			load_ray<PASS, MODE == kWatertight>(a, listed ? a.left[work] : work, a.margin_abs, a.fast_scene != 0, r);
+			load_ray<PASS, MODE == kWatertight>(a, listed ? a.left[work] : work, a.margin_abs, a.reach, r);
 			active = r.mine;
 			const uint64_t left = __ballot(!active && g == 0u);
 			if (left != 0ull && !full) {  // to the second pass: one atomic for the wave's groups
@@ -1207,8 +1197,8 @@ hipError_t run_trace(const Bvh8 &b, const TraceParams &p, const float *rays, uin
 	a.n_tiles = batch ? batch->n_tiles : 0u;
 	a.scene_info = batch ? batch->info : nullptr;
 	if (batch && (seeds || b.n_nodes < batch->n_scenes || !batch->tiles || !batch->info)) return hipErrorInvalidValue;
-	a.fast_scene = 1;
-	for (int k = 0; k < 6; ++k) a.fast_scene &= std::fabs(b.scene_box[k]) < 0x1p60f ? 1 : 0;
+	a.reach = 0.0f;
+	for (int k = 0; k < 6; ++k) a.reach = std::max(a.reach, std::fabs(b.scene_box[k]));
 
 	if (clear) hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, st, a.counter, static_cast<int>(kCounters));
 	hipEvent_t e0 = nullptr, e1 = nullptr;
