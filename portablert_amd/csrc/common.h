@@ -311,16 +311,23 @@ __host__ __device__ inline bool ray_in_range(const float o[3], const float d[3],
 // few parts in a hundred more for the grid's rounding: len_k knows nothing of those axes, so a box
 // thin on axis k near coordinate 0 would end before the hit. Such a ray is fast only if |o_k| alone
 // covers them (2^40, to spare).
-__host__ __device__ inline bool one_fma_ray(const float o[3], const float d[3], const float inv[3], float reach) {
-	float inv_max = 0.0f, o_max = 0.0f;
+// `exact` (no distance culling: every input as the reference has it), and with a zero component always:
+// the margin must also hold what denormal products lose, up to 2^-141 of t (255 steps of 2^-150 and the
+// single roundings): 2^-18 |1/d_k| len_k does where |1/d_k| >= 2^-4, since len_k >= 255 * 2^-126, or
+// where |o_k / d_k| >= 2^-118.
+__host__ __device__ inline bool one_fma_ray(const float o[3], const float d[3], const float inv[3], float reach,
+                                            bool exact) {
+	float inv_max = 0.0f, o_max = 0.0f, flat = __builtin_inff(), low = __builtin_inff();
 	for (int k = 0; k < 3; ++k) {
-		if (d[k] != 0.0f) inv_max = fmaxf(inv_max, fabsf(inv[k]));
-		o_max = fmaxf(o_max, fabsf(o[k]));
+		const float a = fabsf(inv[k]), b = fabsf(o[k]);
+		const bool zero = d[k] == 0.0f;
+		inv_max = zero ? inv_max : fmaxf(inv_max, a);
+		o_max = fmaxf(o_max, b);
+		flat = zero ? fminf(flat, 0x1p40f * b) : flat;
+		low = zero ? low : fminf(low, fmaxf(0x1p4f * a, 0x1p118f * (a * b)));
 	}
-	const float t_max = (reach + o_max) * inv_max;
-	bool ok = d[0] != 0.0f;
-	for (int k = 1; k < 3; ++k) ok &= d[k] != 0.0f || 0x1p40f * fabsf(o[k]) >= t_max;
-	return ok;
+	exact |= flat < __builtin_inff();
+	return d[0] != 0.0f && flat >= (reach + o_max) * inv_max && (!exact || low >= 1.0f);
 }
 
 // Keep the better of (t, id): smaller t, equal finite t resolved to the lower id. NaN and +inf

@@ -6,7 +6,7 @@ import pytest
 import oracle
 import portablert_amd as prt
 from helpers import assert_same
-from test_one_fma_rays import THIN, squeezed, swap_yz
+from test_one_fma_rays import THIN, huge_directions, squeezed, swap_yz
 
 pytestmark = pytest.mark.gpu
 
@@ -52,6 +52,20 @@ def test_squeezed_scene(gpu_ctx, n_rays):
     """Many such triangles together, by eight lanes a ray and by one, without distance culling."""
     tris, rays = squeezed(np.random.default_rng(7), 300)
     rays = np.resize(rays, (n_rays, 6))
+    want = oracle.brute(tris, rays)
+    gpu_ctx.set_tris(tris)
+    try:
+        for waves in (0, 16):
+            options(gpu_ctx, cull=0, waves_per_cu=waves)
+            assert_same(gpu_ctx.nearest_hits(rays, FULL), want, what=f"waves={waves}")
+    finally:
+        options(gpu_ctx)
+
+
+def test_huge_directions_without_culling(gpu_ctx):
+    """t down to the denormals, where the one-fma test's margins end: the reference formula's rays."""
+    tris, rays = huge_directions(np.random.default_rng(11), 400)
+    rays = np.resize(rays, (8000, 6))
     want = oracle.brute(tris, rays)
     gpu_ctx.set_tris(tris)
     try:

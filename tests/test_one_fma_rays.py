@@ -14,11 +14,11 @@ F = np.float32
 
 SRC = """
 #include "common.h"
-extern "C" void one_fma(const float *rays, const float *reach, int n, unsigned char *fast) {
+extern "C" void one_fma(const float *rays, const float *reach, int n, int exact, unsigned char *fast) {
 	for (int i = 0; i < n; ++i) {
 		const float *o = rays + 6 * i, *d = o + 3;
 		const float inv[3] = {1.0f / d[0], 1.0f / d[1], 1.0f / d[2]};
-		fast[i] = prt::ray_in_range(o, d, inv, reach[i]) && prt::one_fma_ray(o, d, inv, reach[i]);
+		fast[i] = prt::ray_in_range(o, d, inv, reach[i]) && prt::one_fma_ray(o, d, inv, reach[i], exact);
 	}
 }
 """
@@ -33,10 +33,10 @@ def one_fma(tmp_path_factory):
                     "-I" + build.CSRC, str(src), "-o", str(so)], check=True)
     lib = ctypes.CDLL(str(so))
 
-    def f(rays, reach):
+    def f(rays, reach, exact=True):
         rays, reach = np.ascontiguousarray(rays, F), np.ascontiguousarray(reach, F)
         out = np.zeros(len(rays), np.uint8)
-        lib.one_fma(*(a.ctypes.data_as(ctypes.c_void_p) for a in (rays, reach)), len(rays),
+        lib.one_fma(*(a.ctypes.data_as(ctypes.c_void_p) for a in (rays, reach)), len(rays), exact,
                     out.ctypes.data_as(ctypes.c_void_p))
         return out.astype(bool)
     return f
@@ -77,9 +77,9 @@ def reference_hits(tris, rays):
     return np.array([oracle.brute(t, r)["t"][0] < np.inf for t, r in zip(tris, rays)])
 
 
-def check(one_fma, tris, rays):
+def check(one_fma, tris, rays, exact=False):
     tris, rays = np.asarray(tris, F), np.asarray(rays, F)
-    fast = one_fma(rays, np.abs(tris).max(1))
+    fast = one_fma(rays, np.abs(tris).max(1), exact)
     hit = reference_hits(tris, rays)
     assert hit.mean() > 0.2  # the inputs reach their triangles
     lost = fast & hit & ~enters(tris, rays)
@@ -139,6 +139,23 @@ def test_squeezed_triangles(one_fma):
     check(one_fma, *squeezed(np.random.default_rng(1), 20000))
 
 
+def huge_directions(rng, n):
+    """Rays of lengths 1e8 to 1e36 at triangles of 1e-32 to 1: t from ordinary to denormal."""
+    size = 10.0 ** rng.uniform(-32, 0, (n, 1))
+    v = (rng.uniform(-1, 1, (n, 9)) * size).astype(F)
+    w = rng.dirichlet((1, 1, 1), n)[:, :, None]
+    at = (v.reshape(n, 3, 3).astype(np.float64) * w).sum(1)
+    d = rng.normal(size=(n, 3))
+    d[rng.random(n) < .2, 1] = 0
+    d[rng.random(n) < .2, 2] = 0
+    o = at - d * size * 10.0 ** rng.uniform(-2, 2, (n, 1))
+    return v, np.concatenate([o, d * 10.0 ** rng.uniform(8, 36, (n, 1))], 1).astype(F)
+
+
+def test_huge_directions(one_fma):
+    check(one_fma, *huge_directions(np.random.default_rng(3), 20000), exact=True)
+
+
 def test_ordinary_rays_stay_fast(one_fma):
     """Parallel rays and the centre lines of a camera over a scene of ordinary proportions take the
     one-fma test, but for those with the coordinate 0 itself on the zero axis."""
@@ -146,6 +163,8 @@ def test_ordinary_rays_stay_fast(one_fma):
     rays = rng.uniform(-2, 2, (4000, 6)).astype(F)
     rays[np.arange(4000) % 2 == 0, 4] = 0
     rays[np.arange(4000) % 3 == 0, 5] = 0
+    assert one_fma(rays, np.full(4000, 30, F)).all()
+    rays[:, 3:] *= 1000
     assert one_fma(rays, np.full(4000, 30, F)).all()
     rays[:, 3] = 0
     assert not one_fma(rays, np.full(4000, 30, F)).any()
