@@ -45,7 +45,7 @@ enum : int {
 	M_NCULL = 1,       // triangles flagged by cull_unsafe (never culled by distance)
 	M_PTILES = 2,      // clustering: tiles of the cluster list a step reads, by parity of the step,
 	M_PSTRIDE = 4,     // and how far apart they are
-	M_PHELD = 6,       // clustering: 0, or 1 + the list buffer that holds the last kTailMax clusters
+	M_PHELD = 6,       // clustering: the step that found at most kTailMax clusters (held_by), or 0
 	M_PDONE = 7,       // clustering: finished
 	M_LCNT = 8,        // per BVH8 level, 64 bits: its nodes, and the triangles of the level above's leaves
 	M_LBASE = M_LCNT + 2 * (kMaxLevels + 2),  // first node of each BVH8 level
@@ -824,6 +824,7 @@ struct PlocArgs {
 	uint32_t *cnt_out;
 	uint32_t *scan_out;       // a copy of cnt_out (0 past the last tile) to be scanned, or null
 	uint32_t *misc;
+	uint32_t step;            // from 0
 	int parity;               // of the step: reads buffer `parity`, writes the other
 	uint32_t tiles_max;       // tiles of the first step: the scan has one more entry
 };
@@ -877,7 +878,7 @@ __global__ __launch_bounds__(kStepBlock) __attribute__((amdgpu_waves_per_eu(6)))
 	if (!FIRST) {
 		tiles = a.misc[M_PTILES + a.parity];
 		stride = a.misc[M_PSTRIDE + a.parity];
-		if (a.misc[M_PHELD]) return;  // the tail's turn already
+		if (held_before(a.misc[M_PHELD], a.step)) return;  // the tail's turn already
 		if (a.pre) {
 			m = a.scan_in[a.tiles_max] + a.pre[a.tiles_max / kScanSeg];
 		} else {
@@ -913,7 +914,7 @@ __global__ __launch_bounds__(kStepBlock) __attribute__((amdgpu_waves_per_eu(6)))
 			__syncthreads();
 		}
 		if (m <= kTailMax) {
-			if (blockIdx.x == 0 && tid == 0) a.misc[M_PHELD] = 1u + a.parity;
+			if (blockIdx.x == 0 && tid == 0) a.misc[M_PHELD] = held_by(a.step);
 			return;
 		}
 	}
@@ -1077,9 +1078,10 @@ __global__ __launch_bounds__(kTailBlock) void k_ploc_tail(PlocArgs a, uint32_t *
 	if (FIRST) {
 		if (i < m) s.id[i] = n - 1 + i;
 	} else {
-		const uint32_t *list = held == 1u ? a.list_in : a.list_out;
-		const uint32_t *cnt = held == 1u ? a.cnt_in : a.cnt_out;
-		const uint32_t tiles = a.misc[M_PTILES + (held - 1u)], stride = a.misc[M_PSTRIDE + (held - 1u)];
+		const uint32_t buf = held_buffer(held);
+		const uint32_t *list = buf == 0u ? a.list_in : a.list_out;
+		const uint32_t *cnt = buf == 0u ? a.cnt_in : a.cnt_out;
+		const uint32_t tiles = a.misc[M_PTILES + buf], stride = a.misc[M_PSTRIDE + buf];
 		// gather the tiles' clusters in order, a wave per tile in turn
 		m = 0;
 		for (uint32_t t = 0; t < tiles; t += kTailBlock / 64) {
@@ -2039,6 +2041,7 @@ hipError_t build_bvh8(BuildScratch &s, uint64_t n64, const BuildParams &p, Bvh8 
 	// One step, in which buffer step & 1 is read and the other written.
 	auto ploc_args = [&](int par) {
 		const uint64_t list_n = static_cast<uint64_t>(p_tiles) * kStepTile;
+		pa.step = static_cast<uint32_t>(step);
 		pa.parity = par;
 		pa.list_in = lists + par * list_n;
 		pa.list_out = lists + (par ^ 1) * list_n;

@@ -75,6 +75,15 @@ struct BuildScratch {
 	hipEvent_t ev[2] = {nullptr, nullptr};  // build and refit timing
 };
 
+// Clustering: the word that a step sets once at most the tail's clusters are left: 0, or 1 + that
+// step. Its launch sets it while workgroups of the same launch still start, and each of their waves
+// reads it by itself: only what an earlier launch wrote may decide, so that a workgroup's waves agree
+// (on "not 0" some would leave and the others sum tile counts that nobody wrote).
+__host__ __device__ inline uint32_t held_by(uint32_t step) { return step + 1u; }
+__host__ __device__ inline bool held_before(uint32_t held, uint32_t step) { return held != 0u && held <= step; }
+// The list buffer that step read, which holds the clusters.
+__host__ __device__ inline uint32_t held_buffer(uint32_t held) { return (held - 1u) & 1u; }
+
 struct BuildParams {
 	int leaf_size = 3;  // 1..kMaxLeaf
 	int width = 8;      // children per BVH8 node, 2..8 (the node format has 8 slots)

@@ -1,0 +1,20 @@
+"""The clustered build with more workgroups than the chip holds at once, where the clustering ends:
+its last launches start workgroups while the first one reports that few clusters are left."""
+import numpy as np
+import pytest
+
+import oracle
+import portablert_amd as prt
+from helpers import assert_same
+from test_gpu_build import rays_in, soup
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [600001, 1000003, 1900001])
+def test_builds_agree(gpu_ctx, n):
+    tris, rays = soup(n, n), rays_in(64, n)
+    want = oracle.brute(tris, rays)
+    for k in range(3):
+        gpu_ctx.set_tris(tris)
+        assert_same(gpu_ctx.nearest_hits(rays, prt.mask_of(prt.ALL_TAGS)), want, what=f"n={n} build {k}")
