@@ -958,6 +958,10 @@ __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(PASS
 				if (at < static_cast<uint32_t>(kWideStack)) stack[at] = e;
 				else *spilled(at) = e;
 			}
+			// the group's other lanes pop these entries
+			__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+			__builtin_amdgcn_wave_barrier();
+			__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 			sp += hits != 0u ? hits - 1u : 0u;
 			const uint32_t fs = first & 7u;
 			cur = first != kMiss ? child_entry(((fs < 4u ? w1.z : w1.w) >> (8u * (fs & 3u))) & 0xFFu, w1.x, lbase) : kInvalid;
