@@ -1237,7 +1237,30 @@ hipError_t run_trace(const Bvh8 &b, const TraceParams &p, const float *rays, uin
 	return hipSuccess;
 }
 
+// Allocates the counter sets, all 0. Where `st` is being captured they are cleared on a stream of their own:
+// a launch recorded with the graph clears nothing before its first replay, and uncaptured launches
+// and reads of the error flags may come before that.
+hipError_t new_counters(TraceScratch &s, hipStream_t st, bool captured) {
+	constexpr int words = TraceScratch::kSets * TraceScratch::kSetWords;
+	PRT_TRY(s.counter.ensure(sizeof(unsigned long long) * (words + kLeftMax)));
+	hipStream_t own = nullptr;
+	hipError_t e = captured ? hipStreamCreateWithFlags(&own, hipStreamNonBlocking) : hipSuccess;
+	if (e == hipSuccess) {
+		hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, own ? own : st, s.counter.as<unsigned long long>(), words);
+		e = hipGetLastError();
+	}
+	if (own) {
+		if (e == hipSuccess) e = hipStreamSynchronize(own);
+		(void)hipStreamDestroy(own);
+	}
+	if (e != hipSuccess) s.counter.release();
+	else s.clean = true;
+	return e;
+}
+
 }  // namespace
+
+static_assert(static_cast<int>(kCounters) <= TraceScratch::kSetWords, "counter set");
 
 hipError_t trace_bvh8(const Bvh8 &b, TraceScratch &s, const TraceParams &p, const float *rays, uint64_t n,
                       uint32_t mask, void *out, hipStream_t st, float *ms, TraceStats *stats, const SeedArgs *seeds,
@@ -1245,20 +1268,14 @@ hipError_t trace_bvh8(const Bvh8 &b, TraceScratch &s, const TraceParams &p, cons
 	if (n == 0) return hipSuccess;
 	TracePlan pl;
 	PRT_TRY(plan_trace(b, s, p, n, seeds || batch, pl));
-	static_assert(static_cast<int>(kCounters) <= TraceScratch::kSetWords, "counter set");
-	if (!s.counter.ptr) {
-		constexpr int words = TraceScratch::kSets * TraceScratch::kSetWords;
-		PRT_TRY(s.counter.ensure(sizeof(unsigned long long) * (words + kLeftMax)));
-		hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, st, s.counter.as<unsigned long long>(), words);
-		s.clean = true;
-	}
+	hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+	PRT_TRY(hipStreamIsCapturing(st, &cap));
+	const bool captured = cap != hipStreamCaptureStatusNone;
+	if (!s.counter.ptr) PRT_TRY(new_counters(s, st, captured));
 	PRT_TRY(s.spill.ensure(sizeof(uint2) * spill_entries(pl, p)));
 	// Sets 0 and 1 alternate: a launch clears the set of the next one, which saves that one its
 	// clearing kernel (1.3 to 4.3 us). A launch recorded into a graph may be
 	// replayed at any time: it has a set of its own and clears it itself.
-	hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-	PRT_TRY(hipStreamIsCapturing(st, &cap));
-	const bool captured = cap != hipStreamCaptureStatusNone;
 	const int set = captured ? 2 : s.next_set;
 	const bool clear = captured || !s.clean;
 	if (!captured) s.clean = false;
