@@ -169,7 +169,7 @@ struct TraceScratch {
 
 // Error flags of the last launch with `s`, as a device address valid until the launch after it.
 const uint32_t *trace_error_word(const TraceScratch &s);
-// Reads the error flags of the last traversals launched with `s` (synchronises `st`).
+// Reads the error flags of the last traversal that ran with `s` (synchronises `st`).
 hipError_t trace_errors(TraceScratch &s, hipStream_t st, uint32_t *flags);
 
 // Traces n device rays against `b`, writing HitReg records at `out` (device) with the layout

@@ -501,6 +501,15 @@ __device__ __forceinline__ void test_leaf(const TriRec *tris, uint32_t entry, Ra
 	}
 }
 
+// The first workgroup of a launch clears the set of the launch that follows and, since the error flags
+// of all sets are read together as those of the last launch, the flags of the captured launches' set
+// (the last one, just before the list).
+__device__ __forceinline__ void clear_next(const KArgs &a) {
+	if (blockIdx.x != 0 || !a.next) return;
+	if (threadIdx.x < kCounters) a.next[threadIdx.x] = 0ull;
+	else if (threadIdx.x == kCounters) (a.left - TraceScratch::kSetWords)[C_ERR] = 0ull;
+}
+
 // Waves per SIMD the register allocation must allow. Quantized nodes with an 8-entry LDS stack
 // (4 KB per wave): 8 for the plain mode, i.e. at most 64 VGPRs, which it keeps to without a spill;
 // the traversal is partly latency-bound (dependent node fetches) and the extra waves hide more of
@@ -520,7 +529,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<S
 	const uint32_t n_left = PASS == kRest ? flags[1] : 0u;
 	if (PASS == kRest && n_left == 0u) return;
 	const bool listed = PASS == kRest && n_left <= kLeftMax;
-	if (PASS != kRest && blockIdx.x == 0 && threadIdx.x < kCounters && a.next) a.next[threadIdx.x] = 0ull;
+	if (PASS != kRest) clear_next(a);
 	bool told = false;  // the list is full: this wave adds nothing to it any more
 	constexpr bool MULTI = MODE == kSeededMulti, SEEDED = MODE == kSeeded || MULTI, BATCH = MODE == kBatch;
 	__shared__ uint2 lds[S * B];
@@ -829,7 +838,7 @@ __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(PASS
 	uint32_t *flags = reinterpret_cast<uint32_t *>(a.counter + C_ERR);  // [0] errors, [1] rays left to kRest
 	const uint32_t n_left = PASS == kRest ? flags[1] : 0u;
 	if (PASS == kRest && n_left == 0u) return;
-	if (PASS == kFast && blockIdx.x == 0 && threadIdx.x < kCounters && a.next) a.next[threadIdx.x] = 0ull;
+	if (PASS == kFast) clear_next(a);
 	const bool listed = PASS == kRest && n_left <= kLeftMax;
 	const uint64_t n_work = listed ? n_left : a.n_rays;
 	const uint8_t *nodes = static_cast<const uint8_t *>(a.nodes);
@@ -1004,6 +1013,14 @@ __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(PASS
 
 __global__ void k_zero(unsigned long long *p, int n) {
 	if (static_cast<int>(threadIdx.x) < n) p[threadIdx.x] = 0ull;
+}
+
+// Before a captured launch, one wave: its set (the last one) and the error flags of the others.
+__global__ void k_zero_captured(unsigned long long *sets) {
+	constexpr int last = (TraceScratch::kSets - 1) * TraceScratch::kSetWords;
+	const int t = threadIdx.x;
+	if (t < kCounters) sets[last + t] = 0ull;
+	else if (t - kCounters < TraceScratch::kSets - 1) sets[(t - kCounters) * TraceScratch::kSetWords + C_ERR] = 0ull;
 }
 
 template <class Node, int S, int B, int MODE, bool NC, int PASS>
@@ -1276,9 +1293,10 @@ hipError_t trace_bvh8(const Bvh8 &b, TraceScratch &s, const TraceParams &p, cons
 	// Sets 0 and 1 alternate: a launch clears the set of the next one, which saves that one its
 	// clearing kernel (1.3 to 4.3 us). A launch recorded into a graph may be
 	// replayed at any time: it has a set of its own and clears it itself.
-	const int set = captured ? 2 : s.next_set;
-	const bool clear = captured || !s.clean;
-	if (!captured) s.clean = false;
+	const int set = captured ? TraceScratch::kSets - 1 : s.next_set;
+	const bool clear = !captured && !s.clean;
+	if (captured) hipLaunchKernelGGL(k_zero_captured, dim3(1), dim3(64), 0, st, s.set(0));
+	else s.clean = false;
 	s.last_set = set;
 	PRT_TRY(run_trace(b, p, rays, n, mask, out, st, s.set(set), clear, captured ? nullptr : s.set(set ^ 1),
 	                  s.set(TraceScratch::kSets), s.spill.as<uint2>(), pl, ms, stats, seeds, batch));
