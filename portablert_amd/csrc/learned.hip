@@ -189,7 +189,9 @@ constexpr uint64_t kInferChunk = 1u << 24;  // rays per inference launch: 8 Mi r
 
 // The `best` (1 or 4) most likely clusters of n device rays, to c->top4 [n][best].
 hipError_t infer_all(prt_ctx *c, const float *d_rays, uint64_t n, int best, hipStream_t st) {
-	PRT_TRY(c->top4.ensure(4 * best * std::max<uint64_t>(1, n)));
+	// room for four whatever `best` is: a graph that holds a call with one seed keeps the buffer through
+	// a later call with several
+	PRT_TRY(c->top4.ensure(16 * std::max<uint64_t>(1, n)));
 	for (uint64_t f = 0; f < n; f += kInferChunk) {
 		const int rows = static_cast<int>(std::min<uint64_t>(kInferChunk, n - f));
 		uint32_t *out = c->top4.as<uint32_t>() + best * f;

@@ -36,6 +36,35 @@ class Call:
         torch.cuda.synchronize()
 
 
+def test_captured_learned_call_outlives_a_change_of_seeds(gpu_ctx):
+    """A graph with a one-seed learned call replays after an uncaptured call of as many rays with four
+    seeds: the predictions' buffer has not moved."""
+    import torch
+    tris = soup(3000, 31)
+    gpu_ctx.set_tris(tris)
+    prt.learned_setup(gpu_ctx, seed=1)
+    call, stream, graph = Call(tris, 20000, 32), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+
+    def learned():
+        prt.nearest_hits_learned_device(gpu_ctx, call.rays.data_ptr(), call.n, FULL, call.out.data_ptr(),
+                                        stream.cuda_stream)
+    try:
+        learned()
+        call.check(gpu_ctx, "one seed")
+        with torch.cuda.graph(graph, stream=stream, capture_error_mode="relaxed"):
+            learned()
+        for k in range(3):
+            gpu_ctx.set_option("seeds", 4)
+            learned()
+            call.check(gpu_ctx, f"four seeds, before replay {k}")
+            gpu_ctx.set_option("seeds", 1)
+            with torch.cuda.stream(stream):
+                graph.replay()
+            call.check(gpu_ctx, f"replay {k}")
+    finally:
+        gpu_ctx.set_option("seeds", 1)
+
+
 @pytest.mark.parametrize("n", [1000, 120000])
 def test_first_traversal_is_captured(n):
     import torch
