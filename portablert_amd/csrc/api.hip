@@ -60,15 +60,10 @@ int do_build(prt_ctx *c, const float *tris, uint64_t n) {
 	double ms = 0.0;
 	prt::SceneSet one;
 	one.tris = tris;
+	c->has_scene = false;  // until the build is whole, also if it throws
 	hipError_t e = prt::build_bvh8(c->bs, n, c->bp, c->bvh, c->stream, &bad, &ms, &one);
-	if (e != hipSuccess) {
-		c->has_scene = false;
-		return hip_fail(c, e, "BVH build");
-	}
-	if (bad) {
-		c->has_scene = false;
-		return fail(c, PRT_ERR_INPUT, "set_tris: a triangle vertex is not finite");
-	}
+	if (e != hipSuccess) return hip_fail(c, e, "BVH build");
+	if (bad) return fail(c, PRT_ERR_INPUT, "set_tris: a triangle vertex is not finite");
 	c->build_ms = ms;
 	c->has_scene = true;
 	++c->scene_gen;
@@ -216,7 +211,7 @@ static int do_refit(prt_ctx *c, const float *tris) {
 	return PRT_OK;
 }
 
-static int refit_common(prt_ctx *c, const float *tris, uint64_t n, hipMemcpyKind kind) {
+static int refit_any(prt_ctx *c, const float *tris, uint64_t n, hipMemcpyKind kind) {
 	if (!c) return PRT_ERR_ARG;
 	c->err.clear();
 	if (!c->has_scene) return fail(c, PRT_ERR_STATE, "refit called before set_tris");
@@ -233,7 +228,7 @@ static int refit_common(prt_ctx *c, const float *tris, uint64_t n, hipMemcpyKind
 	return do_refit(c, c->bs.tri_in.as<float>());
 }
 
-int prt_mi355x_set_tris(prt_ctx *c, const float *tris, uint64_t n) {
+static int set_tris_host(prt_ctx *c, const float *tris, uint64_t n) {
 	if (!c) return PRT_ERR_ARG;
 	c->err.clear();
 	if (!tris && n) return fail(c, PRT_ERR_ARG, "set_tris: null triangle pointer");
@@ -249,15 +244,7 @@ int prt_mi355x_set_tris(prt_ctx *c, const float *tris, uint64_t n) {
 	return do_build(c, c->bs.tri_in.as<float>(), n);
 }
 
-int prt_mi355x_refit(prt_ctx *c, const float *tris, uint64_t n) {
-	return refit_common(c, tris, n, hipMemcpyHostToDevice);
-}
-
-int prt_mi355x_refit_device(prt_ctx *c, const float *d_tris, uint64_t n) {
-	return refit_common(c, d_tris, n, hipMemcpyDeviceToDevice);
-}
-
-int prt_mi355x_set_tris_device(prt_ctx *c, const float *d_tris, uint64_t n) {
+static int set_tris_dev(prt_ctx *c, const float *d_tris, uint64_t n) {
 	if (!c) return PRT_ERR_ARG;
 	c->err.clear();
 	if (!d_tris && n) return fail(c, PRT_ERR_ARG, "set_tris_device: null triangle pointer");
@@ -272,6 +259,22 @@ int prt_mi355x_set_tris_device(prt_ctx *c, const float *d_tris, uint64_t n) {
 		if (e != hipSuccess) return hip_fail(c, e, "set_tris: copy");
 	}
 	return do_build(c, c->bs.tri_in.as<float>(), n);
+}
+
+int prt_mi355x_set_tris(prt_ctx *c, const float *tris, uint64_t n) {
+	return prt::guarded(c, [&]() -> int { return set_tris_host(c, tris, n); });
+}
+
+int prt_mi355x_set_tris_device(prt_ctx *c, const float *d_tris, uint64_t n) {
+	return prt::guarded(c, [&]() -> int { return set_tris_dev(c, d_tris, n); });
+}
+
+int prt_mi355x_refit(prt_ctx *c, const float *tris, uint64_t n) {
+	return prt::guarded(c, [&]() -> int { return refit_any(c, tris, n, hipMemcpyHostToDevice); });
+}
+
+int prt_mi355x_refit_device(prt_ctx *c, const float *d_tris, uint64_t n) {
+	return prt::guarded(c, [&]() -> int { return refit_any(c, d_tris, n, hipMemcpyDeviceToDevice); });
 }
 
 static int trace_common(prt_ctx *c, const float *d_rays, uint64_t n, uint32_t mask, void *d_out, hipStream_t st) {
