@@ -788,7 +788,9 @@ __device__ __forceinline__ void init_levels(uint32_t *misc, uint32_t tid, uint32
 // left, and the last kTailMax clusters are finished by one workgroup in LDS.
 
 constexpr int kPlocR = 16;
-constexpr int kPlocMaxSteps = 1 << 20;  // more than any input takes: every step merges a pair
+// Steps before a build is given up. A step merges at least one pair, and only one where all areas tie
+// (thousands of equal triangles), which makes a chain deeper than the BVH8 levels allow anyway.
+constexpr int kPlocMaxSteps = 4096;
 constexpr int kStepBlock = 512;
 constexpr int kStepTile = kStepBlock - 2 * kPlocR;  // positions a tile merges: 480 of 512 searched
 constexpr int kStepLoad = kStepTile + 4 * kPlocR;   // positions whose boxes it needs: 544
@@ -2156,7 +2158,7 @@ hipError_t build_bvh8(BuildScratch &s, uint64_t n64, const BuildParams &p, Bvh8 
 	if (!(hm[M_ERR] & 1u)) {
 		if (clustered && !hm[M_PDONE]) {
 			while (!hm[M_PDONE]) {
-				if (step > kPlocMaxSteps) return hipErrorUnknown;
+				if (step >= kPlocMaxSteps) return hipErrorUnknown;
 				for (int k = 0; k < 16; ++k) ploc_step();
 				ploc_tail();
 				PRT_TRY(read_back());
