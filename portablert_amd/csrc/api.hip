@@ -411,7 +411,8 @@ static bool pageable(const void *p) {
 static int nearest_hits_staged(prt_ctx *c, const float *rays, uint64_t n, uint32_t mask, void *out, uint32_t stride,
                                bool *no_memory) {
 	const uint64_t in_bytes = n * 24ull, out_bytes = n * static_cast<uint64_t>(stride);
-	const bool direct = n <= kDirectRays;
+	// a timed traversal works in device memory: its time is not the host link's
+	const bool direct = n <= kDirectRays && !c->time_kernel;
 	auto slice_of = [&](uint64_t bytes) {
 		return direct ? bytes : std::min(kSliceMax, std::max(kSliceMin, (bytes / 4 + 4095) & ~uint64_t{4095}));
 	};
