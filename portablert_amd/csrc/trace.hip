@@ -105,6 +105,7 @@ struct Ray {
 	float abs_margin;  // margin_abs / |d|; infinite: this ray is not culled by distance
 	bool mine;         // this launch traces the ray (Pass)
 	bool odd;          // some 1/d or o is not finite (child_slab)
+	bool line;         // d_x = 0, and the leaf test's error is bounded (child_slab)
 	bool never;        // no triangle can be hit: NaN in origin or direction, or no direction
 };
 
@@ -130,13 +131,17 @@ __device__ __forceinline__ void load_ray(const KArgs &a, uint64_t idx, float mar
 	r.mine = PASS == kFast ? fast || r.never : !(fast || r.never);
 	// margin_abs / |d|, rounded up (1 + 2^-20 covers the reciprocal square root's error). An
 	// infinite margin turns distance culling off for this ray: culling is exact only for rays
-	// with every direction component 0 or within [2^-30, 2^30] (|d|^2 <= 2^60 bounds them above)
-	// and |o| < 2^60 (cull_unsafe in common.h; a zero component makes its products exactly 0, so
-	// the bound there holds); other rays (huge or tiny values) traverse without it.
+	// with every direction component within [2^-30, 2^30] (|d|^2 <= 2^60 bounds them above)
+	// and |o| < 2^60 (cull_unsafe in common.h); other rays (huge or tiny values, zero components)
+	// traverse without it. Rays along an axis meet walls and edges that run along it, where the
+	// determinant is a rounding error and t anything: 0.7% of 4 M such rays through vertices of the
+	// room differed from the reference with culling.
 	const float len2 = r.d[0] * r.d[0] + r.d[1] * r.d[1] + r.d[2] * r.d[2];
-	r.abs_margin = ((a.cull || WT) && in_range && len2 <= 0x1p60f)
+	const bool bounded = (a.cull || WT) && in_range && len2 <= 0x1p60f;
+	r.abs_margin = bounded && !(zero[0] || zero[1] || zero[2])
 	                   ? margin_abs * (__builtin_amdgcn_rsqf(len2) * (1.0f + 0x1p-20f))
 	                   : __builtin_inff();
+	r.line = bounded && zero[0];
 	r.odd = !(__builtin_isfinite(r.inv[0]) && __builtin_isfinite(r.inv[1]) && __builtin_isfinite(r.inv[2]) &&
 	          __builtin_isfinite(r.o[0]) && __builtin_isfinite(r.o[1]) && __builtin_isfinite(r.o[2]));
 	if (PASS == kFast) {
@@ -165,19 +170,25 @@ __device__ __forceinline__ float cull_limit(const Ray &r, const KArgs &a) {
 // the box lies on the other axes and also behind the origin (bvh.hpp:210-217 with
 // std::max/std::min argument order). Only the leaf test can reject it, so every box that holds
 // o_x has to pass as far as the leaf test's error reaches: everywhere where that error is not
-// bounded (rays that are not culled by distance, flagged subtrees), else where the ray's line,
-// not only the part ahead, comes within 2^-10 of the coordinates' magnitude. The leaf test's
-// (u, v) place a hit of an unflagged triangle within 5 rho 2^-24 of these lengths, rho as in
-// cull_unsafe, so the pairs covered are those the culling margin covers (rho <= 2^13 / 5); the
-// watertight test's sheared vertices are within 2^-21 of them for every triangle.
+// bounded (without culling, values out of range, flagged subtrees), else where the ray's line, not
+// only the part ahead, comes within 2^-8 of the coordinates' magnitude T = |lo| + |hi| + |o|.
+// That holds at any angle. Let the triangle's vertices have x_i = 0 (vertex 1, at o_x), X0, X2 >= 0 above
+// o_x and D_i the distances of the line from them in the yz plane times |d|. The leaf test's three
+// weights times the determinant are N0 = -X2 D1, N1 = X2 D0 - X0 D2, N2 = X0 D1, computed within c 2^-24
+// (X0 + X2) |d| T, c about 10, N2 within c 2^-24 X0 |d| T; a hit has all three of one sign within
+// that. With X2 >= X0 it follows that |D1| <= c 2^-24 |d| T, the line meets the vertex. Else, r = X2 / X0,
+// either the line crosses the edge from vertex 1 to 2 within c 2^-24 T, or D1 <= c 2^-24 |d| T / r and
+// D2 <= r |d| T: the nearer of the two is within sqrt(c 2^-24) T = 2^-10.3 T at worst. (A search for
+// the worst pair ends at 2^-11.0 T.) The T of a box around the triangle's is at least half of its own.
+// The watertight test's sheared vertices are within 2^-21 of theirs.
 struct SlabRay {
 	float o[3], inv[3];
 	bool odd;   // some 1/d or o is not finite
-	bool line;  // d_x = 0, and the leaf test's error is bounded as above
+	bool line;  // d_x = 0, and the leaf test's error is bounded (not: cull off, values out of range)
 };
 
 __device__ __forceinline__ SlabRay slab_ray(const Ray &r) {
-	return {{r.o[0], r.o[1], r.o[2]}, {r.inv[0], r.inv[1], r.inv[2]}, r.odd, r.d[0] == 0.0f && r.abs_margin < __builtin_inff()};
+	return {{r.o[0], r.o[1], r.o[2]}, {r.inv[0], r.inv[1], r.inv[2]}, r.odd, r.line};
 }
 
 template <bool WIDE = false>
@@ -206,7 +217,7 @@ __device__ __forceinline__ float child_slab(const SlabRay &r, const float lo[3],
 		}
 #pragma unroll
 		for (int k = 1; k < 3; ++k) {
-			const float tol = line ? 0x1p-10f * (fabsf(lo[k]) + fabsf(hi[k]) + fabsf(r.o[k])) : 0.0f;
+			const float tol = line ? 0x1p-8f * (fabsf(lo[k]) + fabsf(hi[k]) + fabsf(r.o[k])) : 0.0f;
 			if (__builtin_isfinite(r.inv[k])) {
 				amin[k] -= tol * fabsf(r.inv[k]);
 				amax[k] += tol * fabsf(r.inv[k]);
