@@ -127,7 +127,9 @@ __device__ __forceinline__ void load_ray(const KArgs &a, uint64_t idx, float mar
 	// With NaN in the origin or the direction every t is NaN, which never wins; without a
 	// direction every determinant is 0 (Moller-Trumbore) or NaN (the watertight test).
 	r.never = nan || (zero[0] && zero[1] && zero[2]);
-	const bool fast = in_range && one_fma_ray(r.o, r.d, r.inv, reach, !a.cull && !WT);
+	bool fast = in_range && !zero[0];
+	const bool exact = !a.cull && !WT;
+	if (fast && (exact || zero[1] || zero[2])) fast = one_fma_ray(r.o, r.d, r.inv, reach, exact);
 	r.mine = PASS == kFast ? fast || r.never : !(fast || r.never);
 	// margin_abs / |d|, rounded up (1 + 2^-20 covers the reciprocal square root's error). An
 	// infinite margin turns distance culling off for this ray: culling is exact only for rays
