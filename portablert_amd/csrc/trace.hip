@@ -193,7 +193,8 @@ __device__ __forceinline__ SlabRay slab_ray(const Ray &r) {
 	return {{r.o[0], r.o[1], r.o[2]}, {r.inv[0], r.inv[1], r.inv[2]}, r.odd, r.line};
 }
 
-template <bool WIDE = false>
+// ODD = false: no lane's ray is odd.
+template <bool WIDE = false, bool ODD = true>
 __device__ __forceinline__ float child_slab(const SlabRay &r, const float lo[3], const float hi[3], float limit,
                                             bool flagged = false) {
 #pragma clang fp contract(off)
@@ -206,7 +207,7 @@ __device__ __forceinline__ float child_slab(const SlabRay &r, const float lo[3],
 		amin[k] = fminf(t1, t2);
 		amax[k] = fmaxf(t1, t2);
 	}
-	if (r.odd) {
+	if (ODD && r.odd) {
 		// 1/d infinite on an axis: a box side through the origin gives NaN in the exact test, and a
 		// box containing the origin's coordinate on that axis is unbounded there.
 		const bool x_in = !__builtin_isfinite(r.inv[0]) && lo[0] <= r.o[0] && r.o[0] <= hi[0];
@@ -456,15 +457,20 @@ static __device__ __forceinline__ void run(const NodeF *nodes, const NodeQ *ncul
 		hi[ax][0] = c.x; hi[ax][1] = c.y; hi[ax][2] = c.z; hi[ax][3] = c.w;
 		hi[ax][4] = d.x; hi[ax][5] = d.y; hi[ax][6] = d.z; hi[ax][7] = d.w;
 	}
+	auto test = [&](auto odd) {
 #pragma unroll
-	for (int k = 0; k < 8; ++k) {
-		const uint32_t meta = ((k < 4 ? h.z : h.w) >> (8 * (k & 3))) & 0xFFu;
-		const float l[3] = {lo[0][k], lo[1][k], lo[2][k]};
-		const float u[3] = {hi[0][k], hi[1][k], hi[2][k]};
-		const float tmin = child_slab<WIDE>(slab_ray(r), l, u, ncull != 0u ? __builtin_inff() : limit, (ncull >> k) & 1u);
-		const bool hit = meta != kMetaEmpty && !__builtin_isnan(tmin);
-		hh.key[k] = hit ? sort_key(tmin, k) : kMiss;
-	}
+		for (int k = 0; k < 8; ++k) {
+			const uint32_t meta = ((k < 4 ? h.z : h.w) >> (8 * (k & 3))) & 0xFFu;
+			const float l[3] = {lo[0][k], lo[1][k], lo[2][k]};
+			const float u[3] = {hi[0][k], hi[1][k], hi[2][k]};
+			const float tmin = child_slab<WIDE, decltype(odd)::value>(slab_ray(r), l, u, ncull != 0u ? __builtin_inff() : limit,
+			                                                          (ncull >> k) & 1u);
+			const bool hit = meta != kMetaEmpty && !__builtin_isnan(tmin);
+			hh.key[k] = hit ? sort_key(tmin, k) : kMiss;
+		}
+	};
+	if (__ballot(r.odd) != 0ull) test(std::true_type());
+	else test(std::false_type());
 	if (ncull != 0u) no_cull_keys(hh.key, ncull);
 	sort8(hh.key);
 }
