@@ -1157,9 +1157,14 @@ hipError_t plan_trace(const Bvh8 &b, TraceScratch &s, const TraceParams &p, uint
 	const uint64_t waves = static_cast<uint64_t>(s.n_cus) * static_cast<uint64_t>(wpc);
 	uint64_t grid64 = (waves * 64 + B - 1) / B;
 	// With at most one ray per launched lane a wave reserves a wave's worth: twice that leaves half of
-	// the waves without work (65,536 room rays 184 -> 138 us, 16,384 169 -> 121 us). Above that the
-	// default of 128 halves the reservations (1 Mi icosphere rays 316 against 406 us).
-	pl.chunk = static_cast<uint32_t>(n <= waves * 64 ? 64 : std::max(64, std::min(1 << 16, p.chunk)));
+	// the waves without work, which costs a ray's chain of visits, so by the tree's depth; the default of
+	// 128 halves the reservations, which cost about 70 ps a ray. 128 against 64, in us: 12 triangles (2 levels)
+	// 32,768 rays 30 / 27, 65,536 38 / 40, 262,144 94 / 114; 400 (5) 131,072 rays 92 / 88, 200,000 114 / 121;
+	// 8,000 (6) 131,072 rays 179 / 158, 200,000 210 / 218; 20,000 (7) 200,000 rays 257 / 251; 100,000 (8)
+	// 262,144 rays 443 / 420; the room (11) 208 / 167 and 263 / 246. Above one ray per lane 128 is the faster
+	// (1 Mi icosphere rays 316 against 406 us).
+	const uint64_t one_each = std::min<uint64_t>(waves * 64, 37500ull * (std::max(2u, b.depth) - 1u));
+	pl.chunk = static_cast<uint32_t>(n <= one_each ? 64 : std::max(64, std::min(1 << 16, p.chunk)));
 	const uint64_t need_threads = (n + 63) / 64 * 64;
 	grid64 = std::max<uint64_t>(1, std::min<uint64_t>(grid64, (need_threads + B - 1) / B));
 	pl.grid = static_cast<uint32_t>(grid64);
