@@ -535,13 +535,16 @@ __device__ __forceinline__ void clear_next(const KArgs &a) {
 // it. The other modes carry more state per lane (seed clusters, scene tiles) and would spill
 // 2 to 5 registers at 64: they run at 7 waves (72 VGPRs, no spill). Spills inside the loop cost far
 // more than a wave of occupancy: the batch step took 8.92 ms at 64 VGPRs with 5 of them, 8.22 ms
-// at 72. A 16-entry stack allows 5 waves by LDS alone. The fp32 node test needs about 100 VGPRs
-// and is left to the compiler (1 = no constraint).
-template <int S, int MODE, int PASS>
-constexpr int kWavesPerEu = PASS == kFast ? (S == 8 ? (MODE == kPlain ? 8 : 7) : 5) : 1;
+// at 72. A 16-entry stack allows 5 waves by LDS alone. The fp32 node test needs 101 VGPRs; held to 96 with
+// 2 spilled, 5 waves instead of 4, 8 M rays take 2.33 ms instead of 2.45 in the room and 1.62 instead of
+// 1.70 over the icosphere (5.49 instead of 5.01 over a soup of 100,000). With never-cull masks, seeds or scenes
+// it would spill more and is left to the compiler (1 = no constraint).
+template <int S, int MODE, bool NC, int PASS>
+constexpr int kWavesPerEu = PASS == kFast ? (S == 8 ? (MODE == kPlain ? 8 : 7) : 5)
+                            : PASS == kAll && !NC && (MODE == kPlain || MODE == kWatertight) ? 5 : 1;
 
 template <class Node, int S, int B, bool COUNT, int MODE, bool NC, int PASS>
-__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<S, MODE, PASS>))) void k_trace(KArgs a) {
+__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<S, MODE, NC, PASS>))) void k_trace(KArgs a) {
 	static_assert(std::is_same<Node, NodeF>::value == (PASS == kAll), "fp32 nodes take one pass");
 	unsigned long long *work = a.counter + (PASS == kRest ? C_WORK_REST : C_WORK);
 	uint32_t *flags = reinterpret_cast<uint32_t *>(a.counter + C_ERR);  // [0] errors, [1] rays left to kRest
