@@ -679,7 +679,7 @@ def main():
         # this workload; the ceiling weights the measured int32 and fp32 issue rates of this GPU by
         # the kernel's instruction mix (gfx950 issues 32-bit integer adds about 1.8x faster than
         # fp32 work).
-        # The counters leave 42% of the instructions unclassified: at the int32 rate they give
+        # The counters leave 43% of the instructions unclassified: at the int32 rate they give
         # the upper bound used as `peak` (frac is then a lower bound), at the fp32 rate the lower
         # bound `peak_lower`
         achieved_valu = vj["sq_insts_valu_per_dispatch"] / (kernel_ms * 1e-3) / 1e9
@@ -712,7 +712,7 @@ def main():
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": traffic,
                      "formula": "achieved = 40 B/ray x 8,388,608 rays / kernel_ms (stream events over the timed "
-                                "steps, the per-step counter reset included); frac = achieved / peak",
+                                "steps, each step's empty second launch included); frac = achieved / peak",
                      "traffic_source": "FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 per launch from "
                                        "profiles/traffic_room.json (committed counters, not this run)"},
         "valu_roofline": valu,

@@ -94,7 +94,10 @@ enum {
  * backend's is_available (src/intersect_hip.cpp:353-372). */
 int prt_mi355x_probe(int *ndev, char *name, size_t cap);
 
-/* Context on device `device`: one HIP stream, the BVH and reusable staging buffers. */
+/* Context on device `device`: one HIP stream, the BVH and reusable staging buffers. Buffers grow with
+ * the largest call and are kept until prt_mi355x_destroy; of pinned host memory, what
+ * prt_mi355x_nearest_hits needs: two pairs of at most 8 MB from its second call on, two pairs of
+ * 24 MB and 1 Mi records after a call of more than 1,048,576 rays. */
 int prt_mi355x_create(int device, prt_ctx **out);
 void prt_mi355x_destroy(prt_ctx *ctx);
 
@@ -108,7 +111,7 @@ int prt_mi355x_device_name(const prt_ctx *ctx, char *buf, size_t cap);
  * Backend::set_tris (backend.hpp:19, intersect_cpu.cpp:12). */
 int prt_mi355x_set_tris(prt_ctx *ctx, const float *tris9, uint64_t n);
 
-/* Same with the triangles already in device memory (read during the call only). The copy runs
+/* Same with the triangles already in device memory (read during the call only). They are read
  * on the context's own stream, which does not wait for other streams: the caller must have
  * completed its writes to d_tris9 (synchronise the stream that wrote them) before the call. */
 int prt_mi355x_set_tris_device(prt_ctx *ctx, const float *d_tris9, uint64_t n);

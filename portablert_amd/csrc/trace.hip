@@ -82,7 +82,8 @@ enum : int {
 };
 
 // Quantized nodes are traversed in two launches: kFast takes the rays of the one-fma node test
-// and leaves the others (d_x = 0, magnitudes out of its range) to kRest. Up to kLeftMax of them are
+// (one_fma_ray) and leaves the others (d_x = 0, a zero axis near coordinate 0, magnitudes out of its
+// range) to kRest. Up to kLeftMax of them are
 // listed; past that kRest goes through all rays again and takes those (a second look at 24 M
 // rays in 382,000 tiles takes 4.8 ms, which a single such ray must not cost). With none its waves
 // end at once. One kernel for both held
@@ -1180,10 +1181,11 @@ hipError_t plan_trace(const Bvh8 &b, TraceScratch &s, const TraceParams &p, uint
 	const bool wide = p.node_format != 0 && p.waves_per_cu <= 0 && !p.count_stats && !several;
 	const uint32_t wide_groups = static_cast<uint32_t>((std::min(n, resident) * 8 + kWideBlock - 1) / kWideBlock);
 	if (wide && n <= (p.leaf_test == 1 ? resident : resident + resident / 2)) pl.wide_grid = wide_groups;
-	// The second pass's reference formula is a longer chain for one lane: parallel rays along y (z for the
-	// icosphere), one lane against eight, in us: 4,096 rays 237 / 113, 448 / 171, 132 / 65; 65,536 rays 365 / 250, 619 /
-	// 350, 303 / 207; 131,072 rays 354 / 318, 687 / 499, 273 / 210; 262,144 rays 488 / 600, 796 / 920, 403 / 388.
-	// Watertight, the room: 4,096 rays 477 / 216, 131,072 rays 632 / 627, 262,144 rays 789 / 1,205.
+	// The second pass's reference formula is a longer chain for one lane, and its rays are not culled: parallel
+	// rays along y (z for the icosphere), one lane against eight, in us, for room, 1.5 M-triangle soup and icosphere:
+	// 4,096 rays 591 / 267, 1,519 / 637, 311 / 163; 65,536 rays 693 / 472, 1,976 / 1,646, 405 / 333; 131,072 rays
+	// 751 / 705, 2,054 / 2,504, 465 / 364; 262,144 rays 873 / 1,309, 2,465 / 5,210, 619 / 723. Watertight, the room:
+	// 4,096 rays 625 / 269, 131,072 rays 790 / 750, 262,144 rays 948 / 1,442.
 	if (wide && n <= 2 * resident) pl.wide_rest = wide_groups;
 	// stack bound: each visited node pushes at most 7 entries, so 7 * depth + 1 suffice
 	pl.max_entries = 7u * std::max(1u, b.depth) + 8u;
